@@ -7,6 +7,7 @@
 #include <new>
 
 #include "capi_common.hpp"
+#include "census.hpp"
 
 namespace mgpm {
 
@@ -493,7 +494,8 @@ int mgpm_dgraph_upload_ex(const mgpm_graph *g, int device, void *stream,
   if (rc) return rc;
   static bool inited = false;
   if (!inited) {
-    if (tc_device_init()) return fail(MGPM_ERR_HIP, "kernel attribute setup");
+    if (tc_device_init() || census_rows_init())
+      return fail(MGPM_ERR_HIP, "kernel attribute setup");
     inited = true;
   }
   std::unique_ptr<mgpm_dgraph> dg(new mgpm_dgraph);

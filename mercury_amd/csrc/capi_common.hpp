@@ -156,13 +156,17 @@ struct CensusGraph {
   // The graph relabelled in DAG order (census_relabel: ids are ranks by
   // degree, then id), its CSR and DAG; every census pass runs on it.
   DevBuf rowptr, col;
-  DevBuf deg, src, drp, dcol, dsrc;
+  DevBuf deg, src, drp, dcol;
+  // The DAG arc of every CSR entry, and the vertices with out-neighbours
+  // grouped by the row passes' classes (sizes in row_count).
+  DevBuf arc, order;
+  int64_t row_count[4] = {0, 0, 0, 0};
   bool pairs_ready = false;
   uint64_t tab_total = 0;  // pair-table slots
   DevBuf tab_off;          // n + 1 slot offsets
   size_t bytes() const {
     return rowptr.bytes + col.bytes + deg.bytes + src.bytes + drp.bytes +
-           dcol.bytes + dsrc.bytes + tab_off.bytes;
+           dcol.bytes + arc.bytes + order.bytes + tab_off.bytes;
   }
 };
 
@@ -174,12 +178,11 @@ struct CensusWork {
   // in flight on larger budgets): the single-query workspace takes 16 GiB,
   // batch lanes and server slots less.
   size_t budget = size_t(16) << 30;
-  DevBuf t, t_csr, tv, small, slab, wedges, touched, k5_slab;
+  DevBuf t, t_csr, tv, small, slab, wedges, touched;
   DevBuf stamp, lo, mask, list, grows, anchors, table;
   size_t bytes() const {
     return t.bytes + t_csr.bytes + tv.bytes + small.bytes + slab.bytes +
-           wedges.bytes + touched.bytes + k5_slab.bytes + stamp.bytes +
-           lo.bytes + mask.bytes + list.bytes + grows.bytes + anchors.bytes +
+           wedges.bytes + touched.bytes + stamp.bytes + lo.bytes + mask.bytes + list.bytes + grows.bytes + anchors.bytes +
            table.bytes;
   }
 };

@@ -54,7 +54,7 @@ constexpr int kMaxCensusDevices = 64;
 
 // Per-caller budgets of the per-workgroup arrays.
 constexpr size_t kCensusC4Budget = size_t(4) << 30;
-constexpr size_t kCensusK5Budget = size_t(8) << 30;
+constexpr size_t kCensusRowBudget = size_t(8) << 30;  // row passes' slabs
 constexpr size_t kCensus5Budget = size_t(8) << 30;  // pair-table layout
 
 // Layout of the small buffer: census cursors, accumulators, pair-pass
@@ -92,11 +92,27 @@ int zero(void *p, size_t bytes, hipStream_t s) {
 
 // Sizes of the workspace for one pattern on one graph.
 struct Need {
-  size_t t = 0, t_csr = 0, tv = 0, slab = 0, wedges = 0, k5 = 0;
+  size_t t = 0, t_csr = 0, tv = 0, slab = 0, wedges = 0;
   size_t stamp = 0, mask = 0, grows = 0, anchors = 0, table = 0;
-  int c4_groups = 0, k5_waves = 0, groups = 0;
-  int64_t k5_len = 0, mask_words = 0, grows_len = 0;
+  int c4_groups = 0, groups = 0;
+  int64_t mask_words = 0, grows_len = 0;
 };
+
+// Slab bytes of the row passes: the classes run one after the other on one
+// slab.  Without class sizes (count null) every class counts n vertices.
+size_t row_slab(const mgpm_dgraph *dg, int passes, int64_t max_out,
+                const int64_t *count) {
+  size_t b = 0;
+  for (int cls = 0; cls < kRowClassCount; ++cls) {
+    const int64_t n = count ? count[cls] : dg->host->n;
+    for (const bool cliques : {false, true})
+      if (cliques ? is_k5(passes) : cls == kRowClassCount - 1)
+        b = std::max(b, rows_slab_bytes(cls, max_out) *
+                            rows_grid(cls, max_out, n, cliques,
+                                      kCensusRowBudget, dg->cus));
+  }
+  return b;
+}
 
 Need need_for(const mgpm_dgraph *dg, int passes, size_t budget) {
   const CsrGraph &G = *dg->host;
@@ -106,21 +122,12 @@ Need need_for(const mgpm_dgraph *dg, int passes, size_t budget) {
   const CensusGraph &cg = dg->census;
   Need k;
   k.t = static_cast<size_t>(m);
-  k.slab = static_cast<size_t>(census_waves(dg->cus)) * cg.max_out;
+  k.slab = row_slab(dg, passes, cg.max_out, cg.row_count);
   if (needs_c4(passes)) {
     const size_t per = static_cast<size_t>(n) * sizeof(uint32_t);
     k.c4_groups = static_cast<int>(std::min<size_t>(
         1024, std::max<size_t>(64, kCensusC4Budget / (2 * per))));
     k.wedges = static_cast<size_t>(k.c4_groups) * n;
-  }
-  if (is_k5(passes)) {
-    k.k5_len = census_k5_slab_len(cg.max_out, cg.max_deg);
-    const size_t per = static_cast<size_t>(k.k5_len) * sizeof(int32_t);
-    const size_t fit = kCensusK5Budget / per;
-    k.k5_waves = static_cast<int>(
-        std::max<size_t>(4, std::min<size_t>(census_waves(dg->cus), fit)) &
-        ~size_t(3));
-    k.k5 = static_cast<size_t>(k.k5_waves) * k.k5_len;
   }
   if (is_full5(passes)) {
     k.t_csr = static_cast<size_t>(nnz);
@@ -181,7 +188,10 @@ int graph_ready(mgpm_dgraph *dg, hipStream_t s) {
   MGPM_HIP(pos.alloc(a1 * sizeof(int64_t)));
   MGPM_HIP(g.drp.alloc((static_cast<size_t>(n) + 1) * sizeof(int64_t)));
   MGPM_HIP(g.dcol.alloc(std::max<int64_t>(m, 1) * sizeof(int32_t)));
-  MGPM_HIP(g.dsrc.alloc(std::max<int64_t>(m, 1) * sizeof(int32_t)));
+  MGPM_HIP(g.arc.alloc(std::max<int64_t>(nnz, 1) * sizeof(uint32_t)));
+  MGPM_HIP(g.order.alloc(std::max<int32_t>(n, 1) * sizeof(int32_t)));
+  DevBuf cls;  // class sizes and fill counters
+  MGPM_HIP(cls.alloc(2 * kRowClassCount * sizeof(unsigned)));
   size_t tb = 0;
   if (dag_scan_bytes(nnz, &tb)) return fail(MGPM_ERR_HIP, "scan size query");
   MGPM_HIP(scan.alloc(std::max<size_t>(tb, 1)));
@@ -202,9 +212,19 @@ int graph_ready(mgpm_dgraph *dg, hipStream_t s) {
   d.out_rowptr[0] = g.drp.as<int64_t>();
   d.out_col[0] = g.dcol.as<int32_t>();
   if (dag_device_build(d, s)) return fail(MGPM_ERR_HIP, "DAG kernel launch failed");
-  if (census_dag_sources(g.drp.as<int64_t>(), n, g.dsrc.as<int32_t>(),
-                         dg->cus, s))
+  int rc = zero(cls.p, cls.bytes, s);
+  if (rc) return rc;
+  unsigned *cnt = cls.as<unsigned>();
+  if (census_rows_arcs(g.rowptr.as<int64_t>(), g.col.as<int32_t>(),
+                       g.src.as<int32_t>(), nnz, g.drp.as<int64_t>(),
+                       g.dcol.as<int32_t>(), g.arc.as<uint32_t>(), dg->cus,
+                       s) ||
+      census_rows_classify(g.drp.as<int64_t>(), n, cnt, cnt + kRowClassCount,
+                           g.order.as<int32_t>(), s))
     return fail(MGPM_ERR_HIP, "census kernel launch failed");
+  unsigned sizes[kRowClassCount];
+  MGPM_HIP(hipMemcpyAsync(sizes, cnt, sizeof(sizes), hipMemcpyDeviceToHost,
+                          s));
   g.max_deg = std::max<int32_t>(G.max_degree(), 1);
   // The host plan knows the largest DAG out-degree (the same DAG).
   g.max_out = std::max<int64_t>(dg->tc.max_out, 1);
@@ -215,7 +235,9 @@ int graph_ready(mgpm_dgraph *dg, hipStream_t s) {
   cg.src.swap(g.src);
   cg.drp.swap(g.drp);
   cg.dcol.swap(g.dcol);
-  cg.dsrc.swap(g.dsrc);
+  cg.arc.swap(g.arc);
+  cg.order.swap(g.order);
+  for (int k = 0; k < kRowClassCount; ++k) cg.row_count[k] = sizes[k];
   cg.max_deg = g.max_deg;
   cg.max_out = g.max_out;
   cg.ready = true;
@@ -230,13 +252,13 @@ CensusArgs args_of(mgpm_dgraph *dg, int passes, CensusWork &w,
   CensusArgs c;
   c.drp = cg.drp.as<int64_t>();
   c.dcol = cg.dcol.as<int32_t>();
-  c.dsrc = cg.dsrc.as<int32_t>();
   c.deg = cg.deg.as<int32_t>();
   c.n = dg->host->n;
   c.m = dg->host->nnz / 2;
   c.t = w.t.as<uint32_t>();
-  c.slab = w.slab.as<int32_t>();
-  c.slab_len = cg.max_out;
+  c.arc = cg.arc.as<uint32_t>();
+  c.order = cg.order.as<int32_t>();
+  c.winlo = std::max<int32_t>(0, c.n - kRowWindow);
   c.cursor = cursor_of(w);
   c.acc = census_acc(w);
   c.rowptr = cg.rowptr.as<int64_t>();
@@ -244,10 +266,6 @@ CensusArgs args_of(mgpm_dgraph *dg, int passes, CensusWork &w,
   c.wedges = w.wedges.as<uint32_t>();
   c.touched = w.touched.as<int32_t>();
   c.c4_groups = k.c4_groups;
-  c.k5_slab = w.k5_slab.as<int32_t>();
-  c.k5_len = k.k5_len;
-  c.max_deg = cg.max_deg;
-  c.k5_waves = k.k5_waves;
   c.full5 = is_full5(passes);
   c.t_csr = w.t_csr.as<uint32_t>();
   c.tv = w.tv.as<unsigned long long>();
@@ -265,6 +283,7 @@ Census5Args args5_of(mgpm_dgraph *dg, CensusWork &w, const Need &k) {
   c.nnz = dg->host->nnz;
   c.drp = cg.drp.as<int64_t>();
   c.dcol = cg.dcol.as<int32_t>();
+  c.arc = cg.arc.as<uint32_t>();
   c.t = w.t.as<uint32_t>();
   c.t_csr = w.t_csr.as<uint32_t>();
   c.tv = w.tv.as<unsigned long long>();
@@ -301,12 +320,11 @@ int work_grow(CensusWork &w, const Need &k, hipStream_t s) {
   };
   if ((rc = grow<uint32_t>(w.t, k.t))) return rc;
   if ((rc = grow<char>(w.small, kSmallBytes))) return rc;
-  if ((rc = grow<int32_t>(w.slab, k.slab))) return rc;
+  if ((rc = grow<char>(w.slab, k.slab))) return rc;
   if (k.wedges) {
     if ((rc = grow_z(w.wedges, k.wedges * 4))) return rc;
     if ((rc = grow<int32_t>(w.touched, k.wedges))) return rc;
   }
-  if (k.k5 && (rc = grow<int32_t>(w.k5_slab, k.k5))) return rc;
   if (k.t_csr) {
     if ((rc = grow<uint32_t>(w.t_csr, k.t_csr))) return rc;
     if ((rc = grow<unsigned long long>(w.tv, k.tv))) return rc;
@@ -332,15 +350,16 @@ uint64_t census_work_bytes(const mgpm_dgraph *dg, int passes,
   if (!dg->census.ready) {
     // The DAG the graph will keep, plus a bound on the workspace.
     const CsrGraph &G = *dg->host;
-    const uint64_t dag = 4ull * G.n + 4ull * G.nnz + 8ull * (G.n + 1) +
+    const uint64_t dag = 8ull * G.n + 8ull * G.nnz + 8ull * (G.n + 1) +
                          8ull * (G.nnz / 2);
     const uint64_t work = is_full5(passes) ? budget + 16ull * G.nnz
                                            : 32ull * G.nnz;
-    return dag + work;
+    return dag + work +
+           row_slab(dg, passes, std::max<int64_t>(dg->tc.max_out, 1), nullptr);
   }
   const Need k = need_for(dg, passes, budget);
-  return 4ull * k.t + kSmallBytes + 4ull * k.slab + 8ull * k.wedges +
-         4ull * k.k5 + 4ull * k.t_csr + 8ull * k.tv + 12ull * k.stamp +
+  return 4ull * k.t + kSmallBytes + k.slab + 8ull * k.wedges +
+         4ull * k.t_csr + 8ull * k.tv + 12ull * k.stamp +
          8ull * k.mask + 8ull * k.grows + 4ull * k.anchors + 8ull * k.table;
 }
 
@@ -430,11 +449,13 @@ int census_enqueue(mgpm_dgraph *dg, int passes, CensusWork &w,
   const Need k = need_for(dg, passes, w.budget);
   CensusArgs c = args_of(dg, passes, w, k);
   int rc;
-  if ((rc = zero(w.t.p, static_cast<size_t>(c.m) * 4, s))) return rc;
   if ((rc = zero(w.small.p, kSmallBytes, s))) return rc;
   const bool f5 = is_full5(passes);
   if (f5 && (rc = zero(w.tv.p, static_cast<size_t>(c.n) * 8, s))) return rc;
-  if (census_launch(c, dg->cus, s))
+  const CensusGraph &cg = dg->census;
+  if (census_rows_launch(c, cg.row_count, cg.max_out, false,
+                         w.slab.as<char>(), kCensusRowBudget, dg->cus, s) ||
+      census_sums_launch(c, dg->cus, s))
     return fail(MGPM_ERR_HIP, "census kernel launch failed");
   Census5Args c5;
   if (f5) {
@@ -444,10 +465,11 @@ int census_enqueue(mgpm_dgraph *dg, int passes, CensusWork &w,
   }
   if (needs_c4(passes) && census_c4_launch(c, s))
     return fail(MGPM_ERR_HIP, "census kernel launch failed");
-  if (is_k5(passes) && census_k5_launch(c, s))
+  if (is_k5(passes) &&
+      census_rows_launch(c, cg.row_count, cg.max_out, true, w.slab.as<char>(),
+                         kCensusRowBudget, dg->cus, s))
     return fail(MGPM_ERR_HIP, "census kernel launch failed");
   if (f5) {
-    const CensusGraph &cg = dg->census;
     if ((rc = zero(w.table.p, cg.tab_total * 8, s))) return rc;
     if (census5_classify_launch(c5, s))
       return fail(MGPM_ERR_HIP, "census kernel launch failed");
@@ -461,7 +483,11 @@ int census_enqueue(mgpm_dgraph *dg, int passes, CensusWork &w,
 int census_combine(int pattern, const unsigned long long *acc,
                    uint64_t *count) {
   const uint64_t pairs_t = acc[kCensusEdgePairs], k4 = acc[kCensusK4];
-  const uint64_t tdeg = acc[kCensusTriDegrees];
+  // Half of a sum kept in two halves of 32 bits, exact modulo 2^64.
+  const unsigned __int128 tdeg2 =
+      static_cast<unsigned __int128>(acc[kCensusTriDegrees]) +
+      (static_cast<unsigned __int128>(acc[kCensusTriDegreesHi]) << 32);
+  const uint64_t tdeg = static_cast<uint64_t>(tdeg2 >> 1);
   if (pattern == MGPM_P1) {
     *count = acc[kCensusDeg3] - tdeg + 2 * pairs_t - 4 * k4;
     return MGPM_OK;
@@ -488,7 +514,7 @@ int census_combine(int pattern, const unsigned long long *acc,
     *count = tdk - 3 * tek + 18 * k5e - 60 * k5;
     return MGPM_OK;
   }
-  const uint64_t tri = acc[kCensusTriangles];
+  const uint64_t tri = acc[kCensusTriangles] / 3;
   const uint64_t k4pend = tdk * kInv3;
   const uint64_t gem = acc[kCensusGem] - 12 * k4;
   const uint64_t w4 = acc[kCensusW4];

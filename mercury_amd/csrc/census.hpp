@@ -1,6 +1,6 @@
-// Subgraph census by triangle enumeration (census_kernels.hip): per-edge
-// triangle counts and the sums from which P1 (induced claws) follows in
-// closed form.
+// Subgraph census (census_rows.hip, census_kernels.hip,
+// census5_kernels.hip): per-edge triangle counts and the sums from which
+// the pattern counts follow in closed form.
 #pragma once
 
 #include <hip/hip_runtime_api.h>
@@ -11,15 +11,18 @@ namespace mgpm {
 
 // Accumulator slots (uint64, zeroed by the caller).
 enum CensusAcc : int {
-  kCensusTriangles = 0,   // triangles
-  kCensusTriDegrees = 1,  // sum over triangles of d(x) + d(y) + d(z) - 6
+  kCensusTriangles = 0,   // sum over edges of t_e: 3 x triangles
+  kCensusTriDegrees = 1,  // sum over edges of t_e (d_x + d_y - 4), low 32
+                          //   bits of each term (the high ones in
+                          //   kCensusTriDegreesHi): twice the sum over
+                          //   triangles of d(x) + d(y) + d(z) - 6
   kCensusK4 = 2,          // 4-cliques
   kCensusDeg3 = 3,        // sum over vertices of C(d, 3)
   kCensusEdgePairs = 4,   // sum over edges of C(t_e, 2)
   kCensusPathPairs = 5,   // sum over edges {x,y} of (d_x - t - 1)(d_y - t - 1)
   kCensusC4 = 6,          // 4-cycles (as subgraphs, not necessarily induced)
   kCensusEdgeTriples = 7, // sum over edges of C(t_e, 3)
-  // census_k5_launch, with k_T = 4-cliques on triangle T:
+  // census_rows_launch with cliques, k_T = 4-cliques on triangle T:
   kCensusTriPairs = 8,    // sum over triangles of C(k_T, 2)
   kCensusTriEdgeK = 9,    // sum over triangles of k_T (t_ab + t_ac + t_bc - 6)
   kCensusTriDegK = 10,    // sum over triangles of k_T (d_a + d_b + d_c - 9)
@@ -31,8 +34,8 @@ enum CensusAcc : int {
   kCensusFork = 15,       // sum over ordered edges (c, x) of
                           //   C(d_c - 1, 2)(d_x - 1) - t_cx (d_c - 2)
   kCensusCricket = 16,    // sum over triangles, vertices of C(d - 2, 2)
-  kCensusBullDeg = 17,    // sum over triangles, vertex pairs of
-                          //   (d_a - 2)(d_b - 2)
+  kCensusBullDeg = 17,    // sum over edges of t_e (d_a - 2)(d_b - 2): over
+                          //   triangles, vertex pairs of (d_a - 2)(d_b - 2)
   kCensusTriS = 18,       // sum over vertices of t_v s_v,
                           //   s_v = sum over neighbours x of (d_x - 1)
   kCensusDp3 = 19,        // sum over edges of C(t_e, 2)(d_a + d_b - 6)
@@ -47,6 +50,7 @@ enum CensusAcc : int {
   kCensusK23e = 27,       // sum over vertex pairs {a,c} of
                           //   E(N(a) ∩ N(c)) (codeg(a,c) - 2)
   kCensusTableMiss = 28,  // pair lookups that found no entry (0)
+  kCensusTriDegreesHi = 29,  // high 32 bits of kCensusTriDegrees' terms
   kCensusSlots = 32
 };
 
@@ -56,35 +60,49 @@ enum CensusAcc : int {
 struct CensusArgs {
   const int64_t *drp = nullptr;  // DAG row offsets (n + 1)
   const int32_t *dcol = nullptr; // DAG column array (m)
-  int32_t *dsrc = nullptr;       // work: source of every DAG arc (m)
   const int32_t *deg = nullptr;  // undirected degrees (n)
   int32_t n = 0;
   int64_t m = 0;
-  uint32_t *t = nullptr;         // per DAG arc: triangles on the edge (zeroed)
-  int32_t *slab = nullptr;       // census_waves() x slab_len ints
-  int64_t slab_len = 0;          // >= the largest DAG out-degree
-  unsigned *cursor = nullptr;    // arc cursor, then vertex cursor (zeroed)
+  uint32_t *t = nullptr;         // per DAG arc: triangles on the edge (out)
+  unsigned *cursor = nullptr;    // 16 queue counters (zeroed)
   unsigned long long *acc = nullptr;  // kCensusSlots (zeroed)
-  // 4-cycle pass (census_c4_launch): undirected CSR (relabelled, rows
-  // sorted), and per workgroup a
-  // dense counter array (zeroed; left zeroed) and a list, n entries each.
+  // Undirected CSR (relabelled, rows sorted), and the DAG arc of each entry.
   const int64_t *rowptr = nullptr;
   const int32_t *col = nullptr;
+  const uint32_t *arc = nullptr;
+  // Vertices with out-neighbours, by class of their number (RowClass), and
+  // the lowest id of the rows' bitmap window.
+  const int32_t *order = nullptr;
+  int32_t winlo = 0;
+  // 4-cycle pass (census_c4_launch): per workgroup a dense counter array
+  // (zeroed; left zeroed) and a list, n entries each.
   uint32_t *wedges = nullptr;
   int32_t *touched = nullptr;
   int c4_groups = 0;
-  // 5-clique pass (census_k5_launch): per wave k5_len ints of slab
-  // (census_k5_slab_len), k5_waves waves; max_deg >= every degree.
-  int32_t *k5_slab = nullptr;
-  int64_t k5_len = 0;
-  int32_t max_deg = 0;
-  int k5_waves = 0;
   // 5-vertex census extras (P2, P3, P5, P6): the terms above marked full5
   // are accumulated only when set; t_csr holds t_e per undirected CSR arc
   // (census_t_csr) for the 4-cycle pass, tv twice the triangles per vertex.
   bool full5 = false;
   const uint32_t *t_csr = nullptr;
   unsigned long long *tv = nullptr;
+};
+
+// One class of vertices of the row passes (census_rows.hip): up to 64,
+// 256 and 704 out-neighbours with their bit rows in LDS, and the rest with
+// rows in the workgroup's slab.
+constexpr int kRowClassCount = 4;
+constexpr int32_t kRowWindow = 65536;  // ids of the bitmap, the highest ones
+
+struct RowArgs {
+  const int32_t *list = nullptr;  // the class's vertices
+  uint32_t count = 0;
+  unsigned *cursor = nullptr;
+  int grab = 1;                   // vertices per queue access
+  char *slab = nullptr;           // per workgroup slab_bytes
+  size_t slab_bytes = 0;
+  uint32_t tri_cap = 0;           // triangles a vertex of the class can have
+  int pcap = 0;                   // out-neighbours it can have
+  int64_t words = 0;              // 64-bit words of row storage
 };
 
 // The pair passes of the 5-vertex census (census5_kernels.hip).  Anchors
@@ -106,6 +124,7 @@ struct Census5Args {
   const int64_t *drp = nullptr;      // DAG
   const int32_t *dcol = nullptr;
   const uint32_t *t = nullptr;       // per DAG arc triangles
+  const uint32_t *arc = nullptr;     // DAG arc of every CSR entry (nnz)
   uint32_t *t_csr = nullptr;         // out: per CSR arc triangles (nnz)
   const unsigned long long *tv = nullptr;  // twice the triangles per vertex
   // Anchor classes: ids grouped by class (n), class sizes and the starts
@@ -138,7 +157,7 @@ struct Census5Args {
 };
 
 // Enqueues t_csr and the per-vertex sums (kCensusTriS, kCensusTv2); needs
-// t and tv from census_launch.
+// t and tv from the row pass and census_sums_launch.
 int census5_flat_launch(const Census5Args &c, int cus, hipStream_t s);
 // The graph relabelled in DAG order: vertex v becomes its rank in the
 // order by (degree, id), so that DAG order is id order -- row v of
@@ -168,26 +187,38 @@ int census5_pairs_launch(const Census5Args &c, hipStream_t s);
 // Per-workgroup bytes of the dense arrays with masks of `words` words.
 size_t census5_group_bytes(int32_t n, int words);
 
-// Waves of the enumeration kernel (slab rows to allocate).
-int census_waves(int cus);
+// Raises the dynamic-LDS limit of the row kernels (once per process).
+int census_rows_init();
 
-// Enqueues the source of every DAG arc into dsrc.  Returns 0, or -1 if
-// the launch failed.
-int census_dag_sources(const int64_t *drp, int32_t n, int32_t *dsrc, int cus,
-                       hipStream_t s);
+// Slab bytes per workgroup of class `cls`, and its workgroups (0 for an
+// empty class) within `budget` bytes of slab, for graphs whose largest DAG
+// out-degree is max_out.  cliques: the pass of that setting.
+size_t rows_slab_bytes(int cls, int64_t max_out);
+int rows_grid(int cls, int64_t max_out, int64_t count, bool cliques,
+              size_t budget, int cus);
 
-// Enqueues the enumeration and the sums (needs dsrc).  Returns 0, or -1 if
-// a launch failed.
-int census_launch(const CensusArgs &c, int cus, hipStream_t s);
+// Enqueues the vertices by class into list (n entries), the class sizes
+// into count (kRowClassCount, with fill zeroed before the call).
+int census_rows_classify(const int64_t *drp, int32_t n, unsigned *count,
+                         unsigned *fill, int32_t *list, hipStream_t s);
 
-// Per-wave slab ints of the 5-clique pass for DAG out-degrees up to
-// max_out and degrees up to max_deg.
-int64_t census_k5_slab_len(int64_t max_out, int64_t max_deg);
+// Enqueues the DAG arc of every CSR entry (src: the entry's row).
+int census_rows_arcs(const int64_t *rowptr, const int32_t *col,
+                     const int32_t *src, int64_t nnz, const int64_t *drp,
+                     const int32_t *dcol, uint32_t *arc, int cus,
+                     hipStream_t s);
 
-// Enqueues the per-triangle 4-clique terms and the 5-clique count
-// (kCensusTriPairs .. kCensusMismatch), with k5_waves waves; needs t[] from
-// census_launch and cursor[2] zero.  Returns 0, or -1 if a launch failed.
-int census_k5_launch(const CensusArgs &c, hipStream_t s);
+// Enqueues one row pass over every class.  cliques = false: t of every arc
+// and kCensusK4; cliques = true (t complete): the per-triangle 4-clique
+// terms and the 5-cliques (kCensusTriPairs .. kCensusMismatch, with full5
+// also kCensusDp2 and kCensusGem).  Each pass has cursors of its own (zero).
+// Returns 0, or -1 if a launch failed.
+int census_rows_launch(const CensusArgs &c, const int64_t *cls_count,
+                       int64_t max_out, bool cliques, char *slab,
+                       size_t budget, int cus, hipStream_t s);
+
+// Enqueues the sums over vertices and edges (needs t).
+int census_sums_launch(const CensusArgs &c, int cus, hipStream_t s);
 
 // Enqueues the 4-cycle count into acc[kCensusC4], with c4_groups
 // workgroups; cursor[1] must be zero.  Returns 0, or -1 if a launch failed.

@@ -114,35 +114,33 @@ __device__ __forceinline__ unsigned long long wg_sum(unsigned long long x,
   return t;
 }
 
-// t per undirected CSR arc: the DAG arc between its ends, found in the
-// DAG row of the lower-ranked end.
+// t per undirected CSR arc, from its DAG arc.
 __global__ void c5_t_csr(Census5Args c) {
   for (int64_t j = int64_t(blockIdx.x) * blockDim.x + threadIdx.x; j < c.nnz;
-       j += int64_t(gridDim.x) * blockDim.x) {
-    const int32_t v = c.src[j], u = c.col[j];
-    const bool vu = above(v, u);
-    const int32_t lo = vu ? v : u, hi = vu ? u : v;
-    const int64_t b = c.drp[lo];
-    const int len = static_cast<int>(c.drp[lo + 1] - b);
-    const int k = lower_bound_p(c.dcol + b, len, hi);
-    c.t_csr[j] = c.t[b + k];
-  }
+       j += int64_t(gridDim.x) * blockDim.x)
+    c.t_csr[j] = c.t[c.arc[j]];
 }
 
-// Sum over vertices of C(t_v, 2), and of t_v s_v as a sum over CSR arcs
-// (v, x) of t_v (d_x - 1).
+// Sums over vertices of C(t_v, 2) and t_v C(d_v - 2, 2), and of t_v s_v as
+// a sum over CSR arcs (v, x) of t_v (d_x - 1).
 __global__ void c5_flat(Census5Args c) {
-  unsigned long long ts = 0, t2 = 0;
+  unsigned long long ts = 0, t2 = 0, crk = 0;
   const int64_t stride = int64_t(gridDim.x) * blockDim.x;
   const int64_t i0 = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
   for (int64_t j = i0; j < c.nnz; j += stride) {
     const unsigned long long tv = c.tv[c.src[j]] >> 1;
     ts += tv * static_cast<unsigned long long>(c.deg[c.col[j]] - 1);
   }
-  for (int64_t v = i0; v < c.n; v += stride) t2 += choose2(c.tv[v] >> 1);
+  for (int64_t v = i0; v < c.n; v += stride) {
+    const unsigned long long tv = c.tv[v] >> 1;  // > 0: degree >= 2
+    t2 += choose2(tv);
+    if (tv) crk += tv * choose2(static_cast<unsigned long long>(c.deg[v]) - 2);
+  }
   ts = wave_sum_u64(ts);
   t2 = wave_sum_u64(t2);
+  crk = wave_sum_u64(crk);
   if (lane64() == 0) {
+    if (crk) atomicAdd(&c.acc[kCensusCricket], crk);
     if (ts) atomicAdd(&c.acc[kCensusTriS], ts);
     if (t2) atomicAdd(&c.acc[kCensusTv2], t2);
   }
