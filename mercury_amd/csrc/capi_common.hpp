@@ -161,12 +161,19 @@ struct CensusGraph {
   // grouped by the row passes' classes (sizes in row_count).
   DevBuf arc, order;
   int64_t row_count[4] = {0, 0, 0, 0};
+  // 4-cycle pass, built when a pattern first needs it: the first entry of
+  // every row in the counters' window, and the owners by kind and class
+  // (light, heavy), one list after the other.
+  bool c4_ready = false;
+  DevBuf c4_win, c4_list;
+  uint32_t c4_count[3][2] = {{0, 0}, {0, 0}, {0, 0}};
   bool pairs_ready = false;
   uint64_t tab_total = 0;  // pair-table slots
   DevBuf tab_off;          // n + 1 slot offsets
   size_t bytes() const {
     return rowptr.bytes + col.bytes + deg.bytes + src.bytes + drp.bytes +
-           dcol.bytes + arc.bytes + order.bytes + tab_off.bytes;
+           dcol.bytes + arc.bytes + order.bytes + c4_win.bytes +
+           c4_list.bytes + tab_off.bytes;
   }
 };
 
@@ -178,11 +185,11 @@ struct CensusWork {
   // in flight on larger budgets): the single-query workspace takes 16 GiB,
   // batch lanes and server slots less.
   size_t budget = size_t(16) << 30;
-  DevBuf t, t_csr, tv, small, slab, wedges, touched;
+  DevBuf t, t_csr, tv, small, slab, wedges;
   DevBuf stamp, lo, mask, list, grows, anchors, table;
   size_t bytes() const {
     return t.bytes + t_csr.bytes + tv.bytes + small.bytes + slab.bytes +
-           wedges.bytes + touched.bytes + stamp.bytes + lo.bytes + mask.bytes + list.bytes + grows.bytes + anchors.bytes +
+           wedges.bytes + stamp.bytes + lo.bytes + mask.bytes + list.bytes + grows.bytes + anchors.bytes +
            table.bytes;
   }
 };

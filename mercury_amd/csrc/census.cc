@@ -64,6 +64,7 @@ constexpr size_t kAccOff = 64;
 constexpr size_t kC5CursorOff = 384;
 constexpr size_t kClsCountOff = 448;
 constexpr size_t kClsFillOff = 480;
+constexpr size_t kC4CursorOff = 512;
 
 // `passes` is a census_passes mask: the triangle pass and the sums always
 // run, the 4-cycle, 5-clique and pair passes on request; the pair passes
@@ -123,11 +124,16 @@ Need need_for(const mgpm_dgraph *dg, int passes, size_t budget) {
   Need k;
   k.t = static_cast<size_t>(m);
   k.slab = row_slab(dg, passes, cg.max_out, cg.row_count);
-  if (needs_c4(passes)) {
-    const size_t per = static_cast<size_t>(n) * sizeof(uint32_t);
-    k.c4_groups = static_cast<int>(std::min<size_t>(
-        1024, std::max<size_t>(64, kCensusC4Budget / (2 * per))));
-    k.wedges = static_cast<size_t>(k.c4_groups) * n;
+  // Heavy 4-cycle owners below the window (before the plan is built: as if
+  // there were some).
+  if (needs_c4(passes) && G.n > kRowWindow &&
+      (!cg.c4_ready || cg.c4_count[2][1])) {
+    const size_t low = static_cast<size_t>(G.n - kRowWindow);
+    const size_t owners = cg.c4_ready ? cg.c4_count[2][1] : low;
+    k.c4_groups = static_cast<int>(std::max<size_t>(
+        1, std::min<size_t>({size_t(dg->cus) * 2, owners,
+                             kCensusC4Budget / (4 * low)})));
+    k.wedges = static_cast<size_t>(k.c4_groups) * low;
   }
   if (is_full5(passes)) {
     k.t_csr = static_cast<size_t>(nnz);
@@ -263,9 +269,9 @@ CensusArgs args_of(mgpm_dgraph *dg, int passes, CensusWork &w,
   c.acc = census_acc(w);
   c.rowptr = cg.rowptr.as<int64_t>();
   c.col = cg.col.as<int32_t>();
+  c.win = cg.c4_win.as<uint32_t>();
+  c.c4_cursor = reinterpret_cast<unsigned *>(w.small.as<char>() + kC4CursorOff);
   c.wedges = w.wedges.as<uint32_t>();
-  c.touched = w.touched.as<int32_t>();
-  c.c4_groups = k.c4_groups;
   c.full5 = is_full5(passes);
   c.t_csr = w.t_csr.as<uint32_t>();
   c.tv = w.tv.as<unsigned long long>();
@@ -321,10 +327,7 @@ int work_grow(CensusWork &w, const Need &k, hipStream_t s) {
   if ((rc = grow<uint32_t>(w.t, k.t))) return rc;
   if ((rc = grow<char>(w.small, kSmallBytes))) return rc;
   if ((rc = grow<char>(w.slab, k.slab))) return rc;
-  if (k.wedges) {
-    if ((rc = grow_z(w.wedges, k.wedges * 4))) return rc;
-    if ((rc = grow<int32_t>(w.touched, k.wedges))) return rc;
-  }
+  if (k.wedges && (rc = grow_z(w.wedges, k.wedges * 4))) return rc;
   if (k.t_csr) {
     if ((rc = grow<uint32_t>(w.t_csr, k.t_csr))) return rc;
     if ((rc = grow<unsigned long long>(w.tv, k.tv))) return rc;
@@ -358,12 +361,67 @@ uint64_t census_work_bytes(const mgpm_dgraph *dg, int passes,
            row_slab(dg, passes, std::max<int64_t>(dg->tc.max_out, 1), nullptr);
   }
   const Need k = need_for(dg, passes, budget);
-  return 4ull * k.t + kSmallBytes + k.slab + 8ull * k.wedges +
+  return 4ull * k.t + kSmallBytes + k.slab + 4ull * k.wedges +
          4ull * k.t_csr + 8ull * k.tv + 12ull * k.stamp +
          8ull * k.mask + 8ull * k.grows + 4ull * k.anchors + 8ull * k.table;
 }
 
 namespace {
+
+// The 4-cycle pass's plan of the graph (once): row offsets of the window,
+// and the owners of every kind and class.
+C4Plan c4_plan_of(const CensusGraph &cg) {
+  C4Plan p;
+  int32_t *at = cg.c4_list.as<int32_t>();
+  for (int k = 0; k < kC4Kinds; ++k) {
+    p.light[k] = cg.c4_count[k][0];
+    p.heavy[k] = cg.c4_count[k][1];
+    p.light_list[k] = at;
+    p.heavy_list[k] = at + p.light[k];
+    at += size_t(p.light[k]) + p.heavy[k];
+  }
+  return p;
+}
+
+int c4_layout(mgpm_dgraph *dg, hipStream_t s) {
+  CensusGraph &cg = dg->census;
+  if (cg.c4_ready) return MGPM_OK;
+  CensusArgs c;
+  c.drp = cg.drp.as<int64_t>();
+  c.rowptr = cg.rowptr.as<int64_t>();
+  c.col = cg.col.as<int32_t>();
+  c.arc = cg.arc.as<uint32_t>();
+  c.n = dg->host->n;
+  c.winlo = std::max<int32_t>(0, c.n - kRowWindow);
+  const size_t n = std::max<size_t>(c.n, 1);
+  DevBuf win, cls, fill;
+  unsigned sizes[2 * kC4Kinds];
+  MGPM_HIP(win.alloc(n * sizeof(uint32_t)));
+  MGPM_HIP(cls.alloc(n + static_cast<size_t>(c.winlo)));
+  MGPM_HIP(fill.alloc(sizeof(sizes)));
+  c.win = win.as<uint32_t>();
+  int rc = zero(fill.p, sizeof(sizes), s);
+  if (rc) return rc;
+  if (census_c4_window(c, win.as<uint32_t>(), s) ||
+      census_c4_classes(c, cls.as<int8_t>(), fill.as<unsigned>(), s))
+    return fail(MGPM_ERR_HIP, "census kernel launch failed");
+  MGPM_HIP(hipMemcpyAsync(sizes, fill.p, sizeof(sizes), hipMemcpyDeviceToHost,
+                          s));
+  MGPM_HIP(hipStreamSynchronize(s));
+  size_t total = 0;
+  for (const unsigned x : sizes) total += x;
+  MGPM_HIP(cg.c4_list.alloc(std::max<size_t>(total, 1) * sizeof(int32_t)));
+  for (int k = 0; k < kC4Kinds; ++k)
+    for (int q = 0; q < 2; ++q) cg.c4_count[k][q] = sizes[2 * k + q];
+  if ((rc = zero(fill.p, sizeof(sizes), s))) return rc;
+  if (census_c4_lists(c, cls.as<int8_t>(), fill.as<unsigned>(),
+                      c4_plan_of(cg), s))
+    return fail(MGPM_ERR_HIP, "census kernel launch failed");
+  MGPM_HIP(hipStreamSynchronize(s));  // the work arrays die here
+  cg.c4_win.swap(win);
+  cg.c4_ready = true;
+  return MGPM_OK;
+}
 
 // The pair-table layout of the graph (once): per anchor, a power of two of
 // slots at least twice the pairs it will hold, from one count pass over
@@ -423,6 +481,7 @@ int pairs_layout(mgpm_dgraph *dg, hipStream_t s) {
 int census_graph_prepare(mgpm_dgraph *dg, hipStream_t s) {
   int rc = graph_ready(dg, s);
   if (rc) return rc;
+  if ((rc = c4_layout(dg, s))) return rc;
   return pairs_layout(dg, s);
 }
 
@@ -440,6 +499,7 @@ int census_prepare(mgpm_dgraph *dg, int passes, CensusWork &w,
                    hipStream_t s) {
   int rc = graph_ready(dg, s);
   if (rc) return rc;
+  if (needs_c4(passes) && (rc = c4_layout(dg, s))) return rc;
   if (is_full5(passes) && (rc = pairs_layout(dg, s))) return rc;
   return work_grow(w, need_for(dg, passes, w.budget), s);
 }
@@ -463,7 +523,8 @@ int census_enqueue(mgpm_dgraph *dg, int passes, CensusWork &w,
     if (census5_flat_launch(c5, dg->cus, s))
       return fail(MGPM_ERR_HIP, "census kernel launch failed");
   }
-  if (needs_c4(passes) && census_c4_launch(c, s))
+  if (needs_c4(passes) &&
+      census_c4_launch(c, c4_plan_of(cg), k.c4_groups, dg->cus, s))
     return fail(MGPM_ERR_HIP, "census kernel launch failed");
   if (is_k5(passes) &&
       census_rows_launch(c, cg.row_count, cg.max_out, true, w.slab.as<char>(),

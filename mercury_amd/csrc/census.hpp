@@ -74,11 +74,12 @@ struct CensusArgs {
   // the lowest id of the rows' bitmap window.
   const int32_t *order = nullptr;
   int32_t winlo = 0;
-  // 4-cycle pass (census_c4_launch): per workgroup a dense counter array
-  // (zeroed; left zeroed) and a list, n entries each.
+  // 4-cycle pass (census_c4.hip): first entry of every row in the window,
+  // queue counters (6, zeroed) and, for heavy owners below the window, per
+  // workgroup a dense counter array (winlo entries, zeroed; left zeroed).
+  const uint32_t *win = nullptr;
+  unsigned *c4_cursor = nullptr;
   uint32_t *wedges = nullptr;
-  int32_t *touched = nullptr;
-  int c4_groups = 0;
   // 5-vertex census extras (P2, P3, P5, P6): the terms above marked full5
   // are accumulated only when set; t_csr holds t_e per undirected CSR arc
   // (census_t_csr) for the 4-cycle pass, tv twice the triangles per vertex.
@@ -220,8 +221,35 @@ int census_rows_launch(const CensusArgs &c, const int64_t *cls_count,
 // Enqueues the sums over vertices and edges (needs t).
 int census_sums_launch(const CensusArgs &c, int cus, hipStream_t s);
 
-// Enqueues the 4-cycle count into acc[kCensusC4], with c4_groups
-// workgroups; cursor[1] must be zero.  Returns 0, or -1 if a launch failed.
-int census_c4_launch(const CensusArgs &c, hipStream_t s);
+// The 4-cycle pass's owners by kind (both ends in the window, the lower
+// one below it, both below) and class; the lists hold light and heavy ids.
+constexpr int kC4Kinds = 3;
+struct C4Plan {
+  uint32_t light[kC4Kinds] = {0, 0, 0}, heavy[kC4Kinds] = {0, 0, 0};
+  int32_t *light_list[kC4Kinds] = {nullptr, nullptr, nullptr};
+  int32_t *heavy_list[kC4Kinds] = {nullptr, nullptr, nullptr};
+};
+struct C4List {
+  const int32_t *list = nullptr;
+  uint32_t count = 0;
+  unsigned *cursor = nullptr;
+};
+
+// Raises the dynamic-LDS limit of the 4-cycle kernels (once per process).
+int census_c4_init();
+// Enqueues the window offsets of the rows (n entries), the classes of the
+// owners (cls: n + winlo entries; class sizes {light, heavy} per kind into
+// fill, zeroed), and, with fill zeroed again, the lists of a plan that
+// points at room for those sizes.
+int census_c4_window(const CensusArgs &c, uint32_t *win, hipStream_t s);
+int census_c4_classes(const CensusArgs &c, int8_t *cls, unsigned *fill,
+                      hipStream_t s);
+int census_c4_lists(const CensusArgs &c, const int8_t *cls, unsigned *fill,
+                    const C4Plan &p, hipStream_t s);
+// Enqueues the 4-cycle count into acc[kCensusC4], with full5 also
+// kCensusBanner and kCensusCycEdgeT; dense_groups: workgroups c.wedges holds
+// arrays for.  Returns 0, or -1 if a launch failed.
+int census_c4_launch(const CensusArgs &c, const C4Plan &p, int dense_groups,
+                     int cus, hipStream_t s);
 
 }  // namespace mgpm
