@@ -124,6 +124,21 @@ int tune_tc(mgpm_dgraph *dg, int reps, mgpm_tune *best, double *best_ms) {
   dg->tc.tuned = true;
   *best = cur;
   *best_ms = cur_ms;
+  // Counts with a NULL tune stay on the hub bitmaps unless the tuned table
+  // plan beats them.
+  dg->hub.off = false;
+  if (tc_hub_wanted(dg)) {
+    std::vector<double> k;
+    for (int i = 0; i < reps + 1; ++i) {
+      uint64_t c = 0;
+      mgpm_stats st;
+      if ((rc = mgpm_tc_count(dg, nullptr, nullptr, &c, &st))) return rc;
+      if (c != want)
+        return fail(MGPM_ERR_INTERNAL, "autotune: candidate count differs");
+      if (i > 0) k.push_back(st.kernel_ms);
+    }
+    dg->hub.off = cur_ms < 0.98 * median(k);
+  }
   return MGPM_OK;
 }
 

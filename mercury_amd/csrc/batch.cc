@@ -182,6 +182,13 @@ int BatchExec::plan(const mgpm_query *q, int nq, uint64_t max_bytes) {
     Planned pq{g, p, 0, -1};
     if (p == MGPM_TC) {
       pq.cost = query_cost(g, p);
+      // The hub plan is kept with the graph, like the census graph it is
+      // made from; without the memory the table plan counts.
+      if (census_ && !g->hub.off && tc_hub_wanted(g)) {
+        const int rc = tc_hub_prepare(g, nullptr);
+        if (rc == MGPM_ERR_NOMEM) (void)hipGetLastError();
+        else if (rc) return rc;
+      }
     } else if (census_) {
       auto it = job_of.find(g);
       if (it == job_of.end()) {
@@ -296,7 +303,12 @@ int BatchExec::enqueue(hipStream_t s, bool copy_back) {
       }
       const int i = u;
       const Planned &qp = queries_[i];
-      if (qp.pattern == MGPM_TC) {
+      if (qp.pattern == MGPM_TC && qp.g->hub.ready && !qp.g->hub.off) {
+        HubOut out;
+        out.result = counters + 2 * i;
+        if (tc_hub_launch(qp.g->hub.plan, out, cus_, ls))
+          return fail(MGPM_ERR_HIP, "triangle kernel launch failed");
+      } else if (qp.pattern == MGPM_TC) {
         TcDevicePlan p = qp.g->tc.dev;
         p.queues = queues + 4 * i;
         p.result = counters + 2 * i;

@@ -195,6 +195,44 @@ int set_device(int device) {
 
 const char *last_error_cstr() { return g_last_error.c_str(); }
 
+// Whether a tune sets a field that the table plan or its launch reads.
+bool tc_knob_set(const mgpm_tune *t) {
+  return t && (t->small_max_deg || t->wave_max_deg || t->block_max_deg ||
+               t->chunk_work || t->grid_blocks || t->group_work ||
+               t->tc_items || t->tc_cursor_min || t->tc_layout ||
+               t->tc_merge_max || t->tc_half_waves);
+}
+
+// What follows a triangle count's launches (enqueued after dg->ev0): the
+// count, and the call's measurements.
+int tc_finish(mgpm_dgraph *dg, hipStream_t s,
+              std::chrono::steady_clock::time_point t0, double prep, int path,
+              uint64_t *count, mgpm_stats *stats) {
+  MGPM_HIP(hipEventRecord(dg->ev1, s));
+  if (path != 3)  // the hub path wrote the count there itself
+    MGPM_HIP(hipMemcpyAsync(dg->pinned, dg->tc.dev.result, 8,
+                            hipMemcpyDeviceToHost, s));
+  MGPM_HIP(hipStreamSynchronize(s));
+  float kms = 0;
+  MGPM_HIP(hipEventElapsedTime(&kms, dg->ev0, dg->ev1));
+  *count = dg->pinned[0];
+  if (stats) {
+    std::memset(stats, 0, sizeof(*stats));
+    stats->kernel_ms = kms;
+    stats->prep_ms = prep;
+    stats->n = static_cast<uint64_t>(dg->host->n);
+    stats->m = static_cast<uint64_t>(dg->host->nnz / 2);
+    stats->m_plus = dg->tc.m_plus;
+    stats->s_plus = dg->tc.s_plus;
+    stats->probes = dg->tc.probes;
+    stats->bytes_alg =
+        8ull * (stats->n + 1) + 20ull * stats->m_plus + 4ull * stats->s_plus;
+    stats->path = path;
+    stats->e2e_ms = ms_since(t0);
+  }
+  return MGPM_OK;
+}
+
 }  // namespace mgpm
 
 using namespace mgpm;
@@ -527,7 +565,8 @@ int mgpm_dgraph_upload_ex(const mgpm_graph *g, int device, void *stream,
 int mgpm_dgraph_footprint(const mgpm_dgraph *dg, uint64_t *bytes) {
   if (!dg || !bytes) return fail(MGPM_ERR_INVALID, "null argument");
   *bytes = dg->tc.bytes() + dg->csr.bytes() + dg->pat.bytes() +
-           dg->dag.bytes() + dg->census.bytes() + dg->scratch.bytes;
+           dg->dag.bytes() + dg->census.bytes() + dg->hub.bytes() +
+           dg->scratch.bytes;
   return MGPM_OK;
 }
 
@@ -557,6 +596,34 @@ int mgpm_tc_count(mgpm_dgraph *dg, const mgpm_tune *tune, void *stream,
   if (rc) return rc;
   hipStream_t s = static_cast<hipStream_t>(stream);
   double prep = 0;
+  // Hub bitmaps where hubs dominate, unless a triangle knob asks for the
+  // table plan; the plan is built on the first such count.  One that cannot
+  // be allocated is skipped (the failed allocation's error is cleared so
+  // that the launch check does not see it).
+  bool hub = !tc_knob_set(tune) && !dg->hub.off && tc_hub_wanted(dg);
+  if (hub && !dg->hub.ready) {
+    const auto tp = std::chrono::steady_clock::now();
+    rc = tc_hub_prepare(dg, s);
+    if (rc == MGPM_ERR_NOMEM) {
+      (void)hipGetLastError();
+      hub = false;
+    } else if (rc) {
+      return rc;
+    }
+    prep = ms_since(tp);
+  }
+  if (hub) {
+    MGPM_HIP(hipEventRecord(dg->ev0, s));
+    // Counters of its own (zero between calls): the count lands in pinned
+    // memory with no fill before it and no copy after it.
+    HubOut out;
+    out.result = dg->hub.own.as<unsigned long long>();
+    out.queue = dg->hub.own.as<unsigned>() + kHubQueueStride;
+    out.host = dg->pinned;
+    if (tc_hub_launch(dg->hub.plan, out, dg->cus, s))
+      return fail(MGPM_ERR_HIP, "triangle kernel launch failed");
+    return tc_finish(dg, s, t0, prep, 3, count, stats);
+  }
   // NULL keeps the resident plan (the defaults, or what mgpm_autotune
   // chose); an explicit tune rebuilds it when its plan knobs differ.
   const TcPlanParams want =
@@ -620,28 +687,7 @@ int mgpm_tc_count(mgpm_dgraph *dg, const mgpm_tune *tune, void *stream,
   MGPM_HIP(hipEventRecord(dg->ev0, s));
   if (tc_device_launch(plan, l, s))
     return fail(MGPM_ERR_HIP, "triangle kernel launch failed");
-  MGPM_HIP(hipEventRecord(dg->ev1, s));
-  MGPM_HIP(hipMemcpyAsync(dg->pinned, dg->tc.dev.result, 8,
-                          hipMemcpyDeviceToHost, s));
-  MGPM_HIP(hipStreamSynchronize(s));
-  float kms = 0;
-  MGPM_HIP(hipEventElapsedTime(&kms, dg->ev0, dg->ev1));
-  *count = dg->pinned[0];
-  if (stats) {
-    std::memset(stats, 0, sizeof(*stats));
-    stats->kernel_ms = kms;
-    stats->prep_ms = prep;
-    stats->n = static_cast<uint64_t>(dg->host->n);
-    stats->m = static_cast<uint64_t>(dg->host->nnz / 2);
-    stats->m_plus = dg->tc.m_plus;
-    stats->s_plus = dg->tc.s_plus;
-    stats->probes = dg->tc.probes;
-    stats->bytes_alg =
-        8ull * (stats->n + 1) + 20ull * stats->m_plus + 4ull * stats->s_plus;
-    stats->path = use_layout ? 2 : 1;
-    stats->e2e_ms = ms_since(t0);
-  }
-  return MGPM_OK;
+  return tc_finish(dg, s, t0, prep, use_layout ? 2 : 1, count, stats);
   MGPM_GUARD_END
 }
 

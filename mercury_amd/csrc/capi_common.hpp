@@ -13,6 +13,7 @@
 #include "mgpm.h"
 #include "pattern_device.hpp"
 #include "tc_device.hpp"
+#include "tc_hub.hpp"
 #include "tc_plan.hpp"
 
 struct mgpm_graph {
@@ -177,6 +178,21 @@ struct CensusGraph {
   }
 };
 
+// The triangle count's hub plan (tc_hub.cc), built on the first count that
+// takes it and kept with the graph.
+struct TcHub {
+  int wanted = -1;  // the rule's answer (-1: not asked yet)
+  bool off = false;  // the autotuner measured a table plan as faster
+  bool ready = false;
+  TcHubPlan plan;
+  DevBuf split, rows, owner, part, bound, start, rest;
+  DevBuf own;  // result and queue of single counts (zero between them)
+  size_t bytes() const {
+    return split.bytes + rows.bytes + owner.bytes + part.bytes + bound.bytes +
+           start.bytes + rest.bytes + own.bytes;
+  }
+};
+
 // Census workspace of one caller (the single-query path of a device, a
 // batch lane, a server slot): grows to the largest query it has served and
 // is reused without allocating.
@@ -259,6 +275,12 @@ int census_combine(int pattern, const unsigned long long *acc,
 // Device bytes of a census workspace for these passes on this graph
 // (before the graph's census DAG exists: a bound that includes it).
 uint64_t census_work_bytes(const mgpm_dgraph *dg, int passes, size_t budget);
+// The census graph alone (relabelled CSR, DAG, arcs), built once.
+int census_graph_ready(mgpm_dgraph *dg, hipStream_t s);
+// Whether triangle counts of the graph go against hub bitmaps unless the
+// caller sets a triangle knob; the plan for it, built once.
+bool tc_hub_wanted(mgpm_dgraph *dg);
+int tc_hub_prepare(mgpm_dgraph *dg, hipStream_t s);
 // Rebuilds the resident triangle plan where it was built (host or device).
 int tc_replan(mgpm_dgraph *dg, const TcPlanParams &params, hipStream_t s);
 // Builds pattern `pattern`'s plan if missing or if `split` (0 = the
@@ -285,6 +307,7 @@ struct mgpm_dgraph {
   mgpm::PatternResident pat;
   mgpm::DagResident dag;
   mgpm::CensusGraph census;            // DAG of the census
+  mgpm::TcHub hub;                     // hub plan of the triangle count
   mgpm::DevBuf scratch;               // queues + result counters
   unsigned long long *pinned = nullptr;  // host mirror of results
   hipEvent_t ev0 = nullptr, ev1 = nullptr;

@@ -478,6 +478,10 @@ int pairs_layout(mgpm_dgraph *dg, hipStream_t s) {
 
 }  // namespace
 
+int census_graph_ready(mgpm_dgraph *dg, hipStream_t s) {
+  return graph_ready(dg, s);
+}
+
 int census_graph_prepare(mgpm_dgraph *dg, hipStream_t s) {
   int rc = graph_ready(dg, s);
   if (rc) return rc;

@@ -265,6 +265,13 @@ int mgpm_server_add_graph(mgpm_server *s, const mgpm_graph *g,
     if ((rc = mgpm_dgraph_upload(g, s->cfg.device, nullptr, &dg))) return rc;
     if (s->cfg.pattern_census >= 0) {
       rc = census_graph_prepare(dg, nullptr);
+      if (!rc && tc_hub_wanted(dg)) {
+        rc = tc_hub_prepare(dg, nullptr);
+        if (rc == MGPM_ERR_NOMEM) {  // the table plan counts triangles
+          (void)hipGetLastError();
+          rc = MGPM_OK;
+        }
+      }
     } else {
       for (int p = MGPM_P1; p <= MGPM_P8 && !rc; ++p)
         rc = pattern_make_resident(dg, nullptr, p);
