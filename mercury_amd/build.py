@@ -40,8 +40,8 @@ LIB_SOURCES = [
     "patterns.cc", "batch.cc", "autotune.cc", "server.cc", "dag.cc",
     "tc_dplan.cc", "tc_hub.cc", "census.cc", "tc_kernels.hip", "tc_hub.hip", "pattern_kernels.hip",
     "dag_kernels.hip", "tc_dplan_kernels.hip", "census_kernels.hip",
-    "census_rows.hip", "census_c4.hip", "census5_kernels.hip",
-    "noalloc.hip",
+    "census_graph.hip", "census_rows.hip", "census_c4.hip",
+    "census5_kernels.hip", "noalloc.hip",
 ]
 CLI_SOURCES = {"tc_challenge": "cli_tc_challenge.cc", "sm": "cli_sm.cc",
                "convert": "cli_convert.cc"}

@@ -3,6 +3,7 @@
 
 #include <hip/hip_runtime_api.h>
 
+#include <algorithm>
 #include <chrono>
 #include <memory>
 #include <string>
@@ -67,6 +68,37 @@ struct DevBuf {
   T *as() const {
     return static_cast<T *>(p);
   }
+};
+
+// Part of a DevBuf.
+struct DevView {
+  void *p = nullptr;
+  template <class T>
+  T *as() const {
+    return static_cast<T *>(p);
+  }
+};
+
+// Lays views out in one allocation: add every view with its size, alloc
+// once (a hipMalloc takes longer than most kernels of a preparation), and
+// the views point into it.
+class DevArena {
+ public:
+  void add(DevView &v, size_t bytes) {
+    views_.push_back({&v, total_});
+    total_ += (std::max<size_t>(bytes, 1) + 255) & ~size_t(255);
+  }
+  hipError_t alloc(DevBuf &mem) {
+    const hipError_t e = mem.alloc(total_);
+    if (e == hipSuccess)
+      for (const auto &v : views_)
+        v.first->p = static_cast<char *>(mem.p) + v.second;
+    return e;
+  }
+
+ private:
+  std::vector<std::pair<DevView *, size_t>> views_;
+  size_t total_ = 0;
 };
 
 // Triangle-count state resident on one device.
@@ -152,15 +184,13 @@ struct DagResident {
 // layout of the 5-vertex census (a function of the graph alone).
 struct CensusGraph {
   bool ready = false;
-  int32_t max_deg = 1;   // largest degree
   int64_t max_out = 1;   // largest DAG out-degree
-  // The graph relabelled in DAG order (census_relabel: ids are ranks by
-  // degree, then id), its CSR and DAG; every census pass runs on it.
-  DevBuf rowptr, col;
-  DevBuf deg, src, drp, dcol;
-  // The DAG arc of every CSR entry, and the vertices with out-neighbours
-  // grouped by the row passes' classes (sizes in row_count).
-  DevBuf arc, order;
+  // The graph relabelled in DAG order (census_build: ids are ranks by
+  // degree, then id), its CSR with the row and the DAG arc of every entry,
+  // and its DAG; every census pass runs on it.  order: the vertices with
+  // out-neighbours grouped by the row passes' classes (sizes in row_count).
+  DevBuf mem;
+  DevView rowptr, col, deg, src, drp, dcol, arc, order;
   int64_t row_count[4] = {0, 0, 0, 0};
   // 4-cycle pass, built when a pattern first needs it: the first entry of
   // every row in the counters' window, and the owners by kind and class
@@ -172,9 +202,7 @@ struct CensusGraph {
   uint64_t tab_total = 0;  // pair-table slots
   DevBuf tab_off;          // n + 1 slot offsets
   size_t bytes() const {
-    return rowptr.bytes + col.bytes + deg.bytes + src.bytes + drp.bytes +
-           dcol.bytes + arc.bytes + order.bytes + c4_win.bytes +
-           c4_list.bytes + tab_off.bytes;
+    return mem.bytes + c4_win.bytes + c4_list.bytes + tab_off.bytes;
   }
 };
 
@@ -185,12 +213,9 @@ struct TcHub {
   bool off = false;  // the autotuner measured a table plan as faster
   bool ready = false;
   TcHubPlan plan;
-  DevBuf split, rows, owner, part, bound, start, rest;
-  DevBuf own;  // result and queue of single counts (zero between them)
-  size_t bytes() const {
-    return split.bytes + rows.bytes + owner.bytes + part.bytes + bound.bytes +
-           start.bytes + rest.bytes + own.bytes;
-  }
+  DevBuf mem;   // everything plan points at, and own
+  DevView own;  // result and queue of single counts (zero between them)
+  size_t bytes() const { return mem.bytes; }
 };
 
 // Census workspace of one caller (the single-query path of a device, a

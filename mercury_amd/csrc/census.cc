@@ -44,7 +44,6 @@
 
 #include "capi_common.hpp"
 #include "census.hpp"
-#include "dag_device.hpp"
 
 namespace mgpm {
 
@@ -167,85 +166,58 @@ int graph_ready(mgpm_dgraph *dg, hipStream_t s) {
   const CsrGraph &G = *dg->host;
   const int64_t nnz = G.nnz;
   const int32_t n = G.n;
-  const int64_t m = nnz / 2;
   if (nnz >= (int64_t(1) << 32))
     return fail(MGPM_ERR_CAPACITY, "census: 2^32 or more arcs");
-  CensusGraph g;
-  MGPM_HIP(g.rowptr.alloc((static_cast<size_t>(n) + 1) * sizeof(int64_t)));
-  MGPM_HIP(g.col.alloc(std::max<int64_t>(nnz, 1) * sizeof(int32_t)));
-  {
-    const size_t rb = census_relabel_bytes(n, nnz);
-    if (rb == 0) return fail(MGPM_ERR_HIP, "sort size query");
-    DevBuf rtmp;
-    MGPM_HIP(rtmp.alloc(rb));
-    if (census_relabel(dg->csr.rowptr.as<int64_t>(),
-                       dg->csr.colidx.as<int32_t>(), n, nnz,
-                       g.rowptr.as<int64_t>(), g.col.as<int32_t>(), rtmp.p,
-                       rb, dg->cus, s))
-      return fail(MGPM_ERR_HIP, "census relabelling failed");
-    MGPM_HIP(hipStreamSynchronize(s));  // rtmp is freed here
-  }
-  DevBuf nd, val, pos, scan;
-  const size_t a1 = static_cast<size_t>(nnz) + 1;
-  MGPM_HIP(g.deg.alloc(std::max<int32_t>(n, 1) * sizeof(int32_t)));
-  MGPM_HIP(nd.alloc(std::max<int32_t>(n, 1) * sizeof(int32_t)));
-  MGPM_HIP(g.src.alloc(std::max<int64_t>(nnz, 1) * sizeof(int32_t)));
-  MGPM_HIP(val.alloc(a1 * sizeof(int64_t)));
-  MGPM_HIP(pos.alloc(a1 * sizeof(int64_t)));
-  MGPM_HIP(g.drp.alloc((static_cast<size_t>(n) + 1) * sizeof(int64_t)));
-  MGPM_HIP(g.dcol.alloc(std::max<int64_t>(m, 1) * sizeof(int32_t)));
-  MGPM_HIP(g.arc.alloc(std::max<int64_t>(nnz, 1) * sizeof(uint32_t)));
-  MGPM_HIP(g.order.alloc(std::max<int32_t>(n, 1) * sizeof(int32_t)));
-  DevBuf cls;  // class sizes and fill counters
-  MGPM_HIP(cls.alloc(2 * kRowClassCount * sizeof(unsigned)));
-  size_t tb = 0;
-  if (dag_scan_bytes(nnz, &tb)) return fail(MGPM_ERR_HIP, "scan size query");
-  MGPM_HIP(scan.alloc(std::max<size_t>(tb, 1)));
-  DagDevice d;
-  d.rowptr = g.rowptr.as<int64_t>();
-  d.col = g.col.as<int32_t>();
-  d.n = n;
-  d.nnz = nnz;
-  d.division = false;
-  d.cus = dg->cus;
-  d.deg = g.deg.as<int32_t>();
-  d.nd = nd.as<int32_t>();
-  d.src = g.src.as<int32_t>();
-  d.val = val.as<int64_t>();
-  d.pos = pos.as<int64_t>();
-  d.scan_tmp = scan.p;
-  d.scan_bytes = tb;
-  d.out_rowptr[0] = g.drp.as<int64_t>();
-  d.out_col[0] = g.dcol.as<int32_t>();
-  if (dag_device_build(d, s)) return fail(MGPM_ERR_HIP, "DAG kernel launch failed");
-  int rc = zero(cls.p, cls.bytes, s);
+  const size_t n1 = static_cast<size_t>(n) + 1;
+  const size_t na = static_cast<size_t>(nnz);
+  DevArena keep, work;
+  keep.add(cg.rowptr, n1 * 8);
+  keep.add(cg.drp, n1 * 8);
+  keep.add(cg.deg, n1 * 4);
+  keep.add(cg.order, n1 * 4);
+  keep.add(cg.col, na * 4);
+  keep.add(cg.src, na * 4);
+  keep.add(cg.arc, na * 4);
+  keep.add(cg.dcol, na / 2 * 4);
+  DevBuf mem, tmp_mem;  // mem becomes cg.mem when it is complete
+  DevView tmp, cls;  // cls: class sizes and fill counters
+  const size_t tb = census_build_bytes(n, nnz);
+  if (tb == 0) return fail(MGPM_ERR_HIP, "sort size query");
+  constexpr size_t kCls = 2 * kRowClassCount * sizeof(unsigned);
+  work.add(tmp, tb);
+  work.add(cls, kCls);
+  MGPM_HIP(keep.alloc(mem));
+  MGPM_HIP(work.alloc(tmp_mem));
+  CensusBuild c;
+  c.in_rowptr = dg->csr.rowptr.as<int64_t>();
+  c.in_col = dg->csr.colidx.as<int32_t>();
+  c.n = n;
+  c.nnz = nnz;
+  c.cus = dg->cus;
+  c.rowptr = cg.rowptr.as<int64_t>();
+  c.drp = cg.drp.as<int64_t>();
+  c.col = cg.col.as<int32_t>();
+  c.src = cg.src.as<int32_t>();
+  c.deg = cg.deg.as<int32_t>();
+  c.dcol = cg.dcol.as<int32_t>();
+  c.arc = cg.arc.as<uint32_t>();
+  c.tmp = tmp.p;
+  c.tmp_bytes = tb;
+  if (census_build(c, s)) return fail(MGPM_ERR_HIP, "census graph build failed");
+  int rc = zero(cls.p, kCls, s);
   if (rc) return rc;
   unsigned *cnt = cls.as<unsigned>();
-  if (census_rows_arcs(g.rowptr.as<int64_t>(), g.col.as<int32_t>(),
-                       g.src.as<int32_t>(), nnz, g.drp.as<int64_t>(),
-                       g.dcol.as<int32_t>(), g.arc.as<uint32_t>(), dg->cus,
-                       s) ||
-      census_rows_classify(g.drp.as<int64_t>(), n, cnt, cnt + kRowClassCount,
-                           g.order.as<int32_t>(), s))
+  if (census_rows_classify(c.drp, n, cnt, cnt + kRowClassCount,
+                           cg.order.as<int32_t>(), s))
     return fail(MGPM_ERR_HIP, "census kernel launch failed");
   unsigned sizes[kRowClassCount];
   MGPM_HIP(hipMemcpyAsync(sizes, cnt, sizeof(sizes), hipMemcpyDeviceToHost,
                           s));
-  g.max_deg = std::max<int32_t>(G.max_degree(), 1);
-  // The host plan knows the largest DAG out-degree (the same DAG).
-  g.max_out = std::max<int64_t>(dg->tc.max_out, 1);
   MGPM_HIP(hipStreamSynchronize(s));  // the work arrays die here
-  cg.rowptr.swap(g.rowptr);
-  cg.col.swap(g.col);
-  cg.deg.swap(g.deg);
-  cg.src.swap(g.src);
-  cg.drp.swap(g.drp);
-  cg.dcol.swap(g.dcol);
-  cg.arc.swap(g.arc);
-  cg.order.swap(g.order);
   for (int k = 0; k < kRowClassCount; ++k) cg.row_count[k] = sizes[k];
-  cg.max_deg = g.max_deg;
-  cg.max_out = g.max_out;
+  // The triangle plan knows the largest DAG out-degree (the same DAG).
+  cg.max_out = std::max<int64_t>(dg->tc.max_out, 1);
+  cg.mem.swap(mem);
   cg.ready = true;
   return MGPM_OK;
 }

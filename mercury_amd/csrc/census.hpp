@@ -54,9 +54,30 @@ enum CensusAcc : int {
   kCensusSlots = 32
 };
 
-// The census runs on the graph relabelled in DAG order (census_relabel):
+// The census runs on the graph relabelled in DAG order (census_build):
 // rank is id, so "ranked below v" is "id below v", every CSR row is sorted
 // with the vertices below its own first, and the DAG rows are the tails.
+//
+// Its construction (census_graph.hip): from the CSR (in_rowptr, in_col) the
+// relabelled CSR (rowptr n + 1, col nnz, the row of every entry src nnz), the
+// degrees, the DAG (drp n + 1, dcol nnz / 2) and the DAG arc of every entry
+// (nnz); tmp holds census_build_bytes.  Returns 0, or -1 if a launch, scan
+// or sort failed.
+struct CensusBuild {
+  const int64_t *in_rowptr = nullptr;
+  const int32_t *in_col = nullptr;
+  int32_t n = 0;
+  int64_t nnz = 0;
+  int cus = 256;
+  int64_t *rowptr = nullptr, *drp = nullptr;
+  int32_t *col = nullptr, *src = nullptr, *deg = nullptr, *dcol = nullptr;
+  uint32_t *arc = nullptr;
+  void *tmp = nullptr;
+  size_t tmp_bytes = 0;
+};
+size_t census_build_bytes(int32_t n, int64_t nnz);  // 0: query failed
+int census_build(const CensusBuild &c, hipStream_t s);
+
 struct CensusArgs {
   const int64_t *drp = nullptr;  // DAG row offsets (n + 1)
   const int32_t *dcol = nullptr; // DAG column array (m)
@@ -160,19 +181,6 @@ struct Census5Args {
 // Enqueues t_csr and the per-vertex sums (kCensusTriS, kCensusTv2); needs
 // t and tv from the row pass and census_sums_launch.
 int census5_flat_launch(const Census5Args &c, int cus, hipStream_t s);
-// The graph relabelled in DAG order: vertex v becomes its rank in the
-// order by (degree, id), so that DAG order is id order -- row v of
-// (out_rowptr, out_col) is sorted, its first d(v) - d+(v) entries lie
-// below v and the rest is N+(v).  Every census sum is a count of subgraphs,
-// the same on either labelling.  One stable sort of the vertices by degree
-// gives the ranks, one sort of the arcs by (rank of the row, rank of the
-// head) the rows.  out_rowptr holds n + 1, out_col nnz words; tmp holds
-// census_relabel_bytes(n, nnz) bytes.  Returns 0, or -1 if a launch, scan
-// or sort failed.
-size_t census_relabel_bytes(int32_t n, int64_t nnz);
-int census_relabel(const int64_t *rowptr, const int32_t *col, int32_t n,
-                   int64_t nnz, int64_t *out_rowptr, int32_t *out_col,
-                   void *tmp, size_t tmp_bytes, int cus, hipStream_t s);
 // Enqueues the pair-table count pass (tab_cap, from zeroed stamps); the
 // caller scans tab_cap into tab_off and sizes the table from tab_off[n].
 int census5_table_count_launch(const Census5Args &c, hipStream_t s);
@@ -202,12 +210,6 @@ int rows_grid(int cls, int64_t max_out, int64_t count, bool cliques,
 // into count (kRowClassCount, with fill zeroed before the call).
 int census_rows_classify(const int64_t *drp, int32_t n, unsigned *count,
                          unsigned *fill, int32_t *list, hipStream_t s);
-
-// Enqueues the DAG arc of every CSR entry (src: the entry's row).
-int census_rows_arcs(const int64_t *rowptr, const int32_t *col,
-                     const int32_t *src, int64_t nnz, const int64_t *drp,
-                     const int32_t *dcol, uint32_t *arc, int cus,
-                     hipStream_t s);
 
 // Enqueues one row pass over every class.  cliques = false: t of every arc
 // and kCensusK4; cliques = true (t complete): the per-triangle 4-clique

@@ -22,12 +22,11 @@
 //     |N+(x) ∩ N(p) ∩ N(q)| (codeg(p, q) - 2) of K2,3+e, codeg from the
 //     table (x lies below p and q, so the pair is there).
 // G[N+(a)] is held as adjacency bit rows, in LDS for d+ up to 512.  The
-// passes run on the census graph, relabelled in DAG order (census_relabel):
+// passes run on the census graph, relabelled in DAG order (census_build):
 // ids compare as ranks, and each sorted row lists the vertices below its
 // own first, then N+.
 #include <hip/hip_runtime.h>
 
-#include <hipcub/device/device_radix_sort.hpp>
 #include <hipcub/device/device_scan.hpp>
 
 #include <algorithm>
@@ -44,7 +43,7 @@ constexpr int kT = 256;  // threads per workgroup
 constexpr int kTW = kT / 64;
 
 // b is ranked above a in DAG order: the census graph is relabelled in that
-// order (census_relabel), so the larger id.
+// order (census_build), so the larger id.
 __device__ __forceinline__ bool above(int32_t a, int32_t b) { return b > a; }
 
 template <class P>
@@ -500,108 +499,6 @@ __global__ __launch_bounds__(kT) void c5_outnb(Census5Args c, int cls) {
   if (threadIdx.x == 0 && w4) atomicAdd(&c.acc[kCensusW4], w4);
 }
 
-// Relabelling in DAG order (census_relabel): degrees and ids, then ranks.
-__global__ void c5_degrees(const int64_t *__restrict__ rowptr, int32_t n,
-                           uint32_t *__restrict__ deg,
-                           uint32_t *__restrict__ ids) {
-  for (int64_t v = int64_t(blockIdx.x) * blockDim.x + threadIdx.x; v < n;
-       v += int64_t(gridDim.x) * blockDim.x) {
-    deg[v] = static_cast<uint32_t>(rowptr[v + 1] - rowptr[v]);
-    ids[v] = static_cast<uint32_t>(v);
-  }
-}
-
-// rank[perm[i]] = i: perm lists the vertices in DAG order; lens[i] = the
-// degree of rank i (lens[n] = 0, for the scan into row pointers).
-__global__ void c5_ranks(const uint32_t *__restrict__ perm,
-                         const uint32_t *__restrict__ dsort, int32_t n,
-                         uint32_t *__restrict__ rank,
-                         int64_t *__restrict__ lens) {
-  for (int64_t i = int64_t(blockIdx.x) * blockDim.x + threadIdx.x; i <= n;
-       i += int64_t(gridDim.x) * blockDim.x) {
-    if (i < n) rank[perm[i]] = static_cast<uint32_t>(i);
-    lens[i] = i < n ? static_cast<int64_t>(dsort[i]) : 0;
-  }
-}
-
-// One key per arc, one wave per row: the rank of its row above the rank
-// of its head (lg bits each).
-__global__ void c5_arc_keys(const int64_t *__restrict__ rowptr,
-                            const int32_t *__restrict__ col, int32_t n,
-                            const uint32_t *__restrict__ rank, int lg,
-                            unsigned long long *__restrict__ keys) {
-  const int lane = lane64();
-  const int64_t nwaves = (int64_t(gridDim.x) * blockDim.x) >> 6;
-  for (int64_t v = (int64_t(blockIdx.x) * blockDim.x + threadIdx.x) >> 6;
-       v < n; v += nwaves) {
-    const unsigned long long r = static_cast<unsigned long long>(rank[v])
-                                 << lg;
-    const int64_t e = rowptr[v + 1];
-    for (int64_t i = rowptr[v] + lane; i < e; i += 64)
-      keys[i] = r | rank[col[i]];
-  }
-}
-
-// The heads' new ids (their ranks), in the sorted order.
-__global__ void c5_arc_heads(const unsigned long long *__restrict__ keys,
-                             int64_t nnz, unsigned long long low,
-                             int32_t *__restrict__ out) {
-  for (int64_t e = int64_t(blockIdx.x) * blockDim.x + threadIdx.x; e < nnz;
-       e += int64_t(gridDim.x) * blockDim.x)
-    out[e] = static_cast<int32_t>(keys[e] & low);
-}
-
-// Layout of census_relabel's scratch: degrees, ids, sorted degrees, the
-// order and the ranks (n words each), the row lengths (n + 1 int64), the
-// arc keys and their sorted copy (nnz u64 each), and the storage of the
-// sorts and the scan.
-struct RelabelTmp {
-  size_t deg = 0, ids = 0, dsort = 0, perm = 0, rank = 0, lens = 0, keys = 0,
-         keys2 = 0, work = 0, work_bytes = 0, total = 0;
-  int lg = 1;  // bits of a vertex id
-};
-
-size_t align256(size_t x) { return (x + 255) & ~size_t(255); }
-
-bool relabel_tmp(int32_t n, int64_t nnz, RelabelTmp *t) {
-  const size_t nv = static_cast<size_t>(std::max<int32_t>(n, 1));
-  const size_t na = static_cast<size_t>(std::max<int64_t>(nnz, 1));
-  t->lg = 1;
-  while (t->lg < 31 && (int64_t(1) << t->lg) < int64_t(n)) ++t->lg;
-  size_t b1 = 0, b2 = 0, b3 = 0;
-  if (hipcub::DeviceRadixSort::SortPairs(
-          nullptr, b1, static_cast<const uint32_t *>(nullptr),
-          static_cast<uint32_t *>(nullptr),
-          static_cast<const uint32_t *>(nullptr),
-          static_cast<uint32_t *>(nullptr), static_cast<int64_t>(nv), 0,
-          32) != hipSuccess)
-    return false;
-  if (hipcub::DeviceRadixSort::SortKeys(
-          nullptr, b2, static_cast<const unsigned long long *>(nullptr),
-          static_cast<unsigned long long *>(nullptr),
-          static_cast<int64_t>(na), 0, 2 * t->lg) != hipSuccess)
-    return false;
-  if (hipcub::DeviceScan::ExclusiveSum(
-          nullptr, b3, static_cast<const int64_t *>(nullptr),
-          static_cast<int64_t *>(nullptr),
-          static_cast<int64_t>(nv + 1)) != hipSuccess)
-    return false;
-  size_t o = 0;
-  t->deg = o;   o += align256(nv * 4);
-  t->ids = o;   o += align256(nv * 4);
-  t->dsort = o; o += align256(nv * 4);
-  t->perm = o;  o += align256(nv * 4);
-  t->rank = o;  o += align256(nv * 4);
-  t->lens = o;  o += align256((nv + 1) * 8);
-  t->keys = o;  o += align256(na * 8);
-  t->keys2 = o; o += align256(na * 8);
-  t->work = o;
-  t->work_bytes = std::max<size_t>(std::max({b1, b2, b3}), 1);
-  o += align256(t->work_bytes);
-  t->total = o;
-  return true;
-}
-
 // Workgroups of a class whose masks take `words` words per vertex: as many
 // as the mask buffer holds slices for, at most c.groups.
 int groups_for(const Census5Args &c, int words) {
@@ -653,60 +550,6 @@ int census5_scan(const unsigned long long *in, unsigned long long *out,
                  hipSuccess
              ? 0
              : -1;
-}
-
-size_t census_relabel_bytes(int32_t n, int64_t nnz) {
-  RelabelTmp t;
-  return relabel_tmp(n, nnz, &t) ? t.total : 0;
-}
-
-int census_relabel(const int64_t *rowptr, const int32_t *col, int32_t n,
-                   int64_t nnz, int64_t *out_rowptr, int32_t *out_col,
-                   void *tmp, size_t tmp_bytes, int cus, hipStream_t s) {
-  if (n < 0) return -1;
-  RelabelTmp t;
-  if (!relabel_tmp(n, nnz, &t) || tmp_bytes < t.total) return -1;
-  char *base = static_cast<char *>(tmp);
-  auto *deg = reinterpret_cast<uint32_t *>(base + t.deg);
-  auto *ids = reinterpret_cast<uint32_t *>(base + t.ids);
-  auto *dsort = reinterpret_cast<uint32_t *>(base + t.dsort);
-  auto *perm = reinterpret_cast<uint32_t *>(base + t.perm);
-  auto *rank = reinterpret_cast<uint32_t *>(base + t.rank);
-  auto *lens = reinterpret_cast<int64_t *>(base + t.lens);
-  auto *keys = reinterpret_cast<unsigned long long *>(base + t.keys);
-  auto *keys2 = reinterpret_cast<unsigned long long *>(base + t.keys2);
-  void *work = base + t.work;
-  const int gv = static_cast<int>(std::min<int64_t>(4096, n / 256 + 1));
-  size_t b = t.work_bytes;
-  if (n > 0) {
-    hipLaunchKernelGGL(c5_degrees, dim3(gv), dim3(256), 0, s, rowptr, n, deg,
-                       ids);
-    // Radix sorts are stable: equal degrees keep id order (DAG order).
-    if (hipcub::DeviceRadixSort::SortPairs(work, b, deg, dsort, ids, perm,
-                                           static_cast<int64_t>(n), 0, 32,
-                                           s) != hipSuccess)
-      return -1;
-  }
-  hipLaunchKernelGGL(c5_ranks, dim3(gv), dim3(256), 0, s, perm, dsort, n,
-                     rank, lens);
-  b = t.work_bytes;
-  if (hipcub::DeviceScan::ExclusiveSum(work, b, lens, out_rowptr,
-                                       static_cast<int64_t>(n) + 1,
-                                       s) != hipSuccess)
-    return -1;
-  if (n > 0 && nnz > 0) {
-    hipLaunchKernelGGL(c5_arc_keys, dim3(std::max(1, cus * 8)), dim3(256), 0,
-                       s, rowptr, col, n, rank, t.lg, keys);
-    b = t.work_bytes;
-    if (hipcub::DeviceRadixSort::SortKeys(work, b, keys, keys2, nnz, 0,
-                                          2 * t.lg, s) != hipSuccess)
-      return -1;
-    const int ga =
-        static_cast<int>(std::min<int64_t>(8192, nnz / 256 + 1));
-    hipLaunchKernelGGL(c5_arc_heads, dim3(ga), dim3(256), 0, s, keys2, nnz,
-                       (1ull << t.lg) - 1ull, out_col);
-  }
-  return hipGetLastError() == hipSuccess ? 0 : -1;
 }
 
 int census5_pairs_launch(const Census5Args &c, hipStream_t s) {

@@ -20,16 +20,34 @@ uint32_t block_count(uint32_t nparts, uint32_t runs, int cus) {
 
 // The degrees of the 65535 highest-degree vertices add up to `num` / `den` of
 // all degrees or more (each arc into a hub counts once there, arcs between
-// hubs twice).
+// hubs twice); with more than 65535 degrees of 4096 and up, by a lower bound.
 bool hubs_hold(const CsrGraph &g, int64_t num, int64_t den) {
-  int32_t top = 0;
-#pragma omp parallel for reduction(max : top)
-  for (int32_t v = 0; v < g.n; ++v) top = std::max(top, g.degree(v));
-  if (den * kHubIds * top < num * g.nnz) return false;
-  std::vector<int64_t> count(static_cast<size_t>(top) + 1, 0);
-  for (int32_t v = 0; v < g.n; ++v) count[g.degree(v)]++;
-  int64_t left = kHubIds, sum = 0;
-  for (int32_t d = top; d > 0 && left > 0; --d) {
+  // Degrees below kFine by value, the rest (on large graphs fewer vertices
+  // than there are hubs) as one bin.
+  constexpr int32_t kFine = 4096;
+  std::vector<int64_t> count(kFine + 1, 0);
+  int64_t high = 0;  // sum of the degrees in the last bin
+#pragma omp parallel
+  {
+    std::vector<int64_t> mine(kFine + 1, 0);
+    int64_t sum = 0;
+#pragma omp for nowait
+    for (int32_t v = 0; v < g.n; ++v) {
+      const int32_t d = g.degree(v);
+      mine[std::min(d, kFine)]++;
+      if (d >= kFine) sum += d;
+    }
+#pragma omp critical
+    {
+      for (int32_t d = 0; d <= kFine; ++d) count[d] += mine[d];
+      high += sum;
+    }
+  }
+  if (count[kFine] >= kHubIds)  // every hub is in the last bin
+    return den * kFine * int64_t(kHubIds) >= num * g.nnz ||
+           den * high * kHubIds >= num * g.nnz * count[kFine];
+  int64_t left = kHubIds - count[kFine], sum = high;
+  for (int32_t d = kFine - 1; d > 0 && left > 0; --d) {
     const int64_t k = std::min<int64_t>(left, count[d]);
     sum += k * d;
     left -= k;
@@ -73,82 +91,70 @@ int tc_hub_prepare(mgpm_dgraph *dg, hipStream_t s) {
   const int64_t nnz = dg->host->nnz, m = nnz / 2;
   const int32_t hublo = std::max<int32_t>(0, n - kHubIds);
   const size_t n1 = static_cast<size_t>(n) + 1;
-  DevBuf split, rowbase, rows, flag, pos, owner, part, bound, start, rest,
-      chunks, tmp, own, total, cost, prefix;
   const uint32_t runs = static_cast<uint32_t>((m + kHubRun - 1) / kHubRun);
-  MGPM_HIP(split.alloc(n1 * 4));
-  MGPM_HIP(chunks.alloc(n1 * 4));
-  MGPM_HIP(rowbase.alloc(n1 * 4));
-  const size_t sb = tc_hub_scan_bytes(n, runs);
-  if (sb == 0) return fail(MGPM_ERR_HIP, "scan size query");
-  MGPM_HIP(tmp.alloc(sb));
   const int64_t *drp = cg.drp.as<int64_t>();
   const int32_t *dcol = cg.dcol.as<int32_t>();
-  if (tc_hub_counts(drp, dcol, n, hublo, split.as<uint32_t>(),
-                    chunks.as<uint32_t>(), s) ||
-      tc_hub_scan(chunks.as<uint32_t>(), rowbase.as<uint32_t>(), n, tmp.p, sb,
-                  s))
-    return fail(MGPM_ERR_HIP, "hub plan kernel launch failed");
-  uint32_t nchunks = 0;
-  MGPM_HIP(hipMemcpyAsync(&nchunks, rowbase.as<uint32_t>() + n, 4,
-                          hipMemcpyDeviceToHost, s));
-  MGPM_HIP(hipStreamSynchronize(s));
-  if (nchunks < 1 || nchunks > m / kHubChunk + n + 1)
-    return fail(MGPM_ERR_INTERNAL, "hub plan: bad row sizes");
   TcHubPlan p;
   p.n = static_cast<uint32_t>(n);
   p.nparts = static_cast<uint32_t>(m);
   p.blocks = block_count(p.nparts, runs, dg->cus);
-  MGPM_HIP(rows.alloc(size_t(nchunks) * kHubChunk * 2));
-  MGPM_HIP(flag.alloc(n1 * 4));
-  MGPM_HIP(pos.alloc(n1 * 4));
-  MGPM_HIP(owner.alloc(static_cast<size_t>(n) * sizeof(HubOwner)));
-  MGPM_HIP(part.alloc(size_t(m) * sizeof(HubPartner)));
-  MGPM_HIP(bound.alloc((size_t(p.blocks) + 1) * 4));
-  MGPM_HIP(start.alloc(size_t(p.blocks) * 4));
-  MGPM_HIP(cost.alloc((size_t(runs) + 1) * 8));
-  MGPM_HIP(prefix.alloc((size_t(runs) + 1) * 8));
-  MGPM_HIP(rest.alloc(static_cast<size_t>(n) * 4));
-  MGPM_HIP(total.alloc(4));
+  // Chunks of all rows: every row rounded up, and the padding chunk.
+  const size_t nchunks = static_cast<size_t>(m) / kHubChunk + n1;
   constexpr size_t kOwnWords = kHubQueueStride + kHubQueueWords;
-  MGPM_HIP(own.alloc(kOwnWords * 4));
-  if (device_zero(total.p, 1, s) || device_zero(own.p, kOwnWords, s) ||
-      tc_hub_fill(cg.rowptr.as<int64_t>(), cg.col.as<int32_t>(),
-                  cg.src.as<int32_t>(), nnz, drp, dcol, cg.arc.as<uint32_t>(),
-                  n, split.as<uint32_t>(), rowbase.as<uint32_t>(), rows.p,
-                  flag.as<uint32_t>(), pos.as<uint32_t>(),
-                  owner.as<HubOwner>(), part.as<HubPartner>(),
-                  rest.as<int32_t>(), total.as<uint32_t>(), tmp.p, sb,
-                  dg->cus, s))
-    return fail(MGPM_ERR_HIP, "hub plan kernel launch failed");
-  MGPM_HIP(hipMemcpyAsync(&p.nrest, total.p, 4, hipMemcpyDeviceToHost, s));
-  MGPM_HIP(hipMemcpyAsync(&p.owners, pos.as<uint32_t>() + n, 4,
-                          hipMemcpyDeviceToHost, s));
-  MGPM_HIP(hipStreamSynchronize(s));
-  if (p.owners == 0) p.blocks = 0;  // no arc follows another: no triangle
+  DevView rows, owner, part, bound, start, rest, split;
+  DevArena keep;
+  keep.add(rows, nchunks * kHubChunk * 2);
+  keep.add(owner, n1 * sizeof(HubOwner));
+  keep.add(part, static_cast<size_t>(m) * sizeof(HubPartner));
+  keep.add(bound, (size_t(p.blocks) + 1) * 4);
+  keep.add(start, (size_t(p.blocks) + 1) * 4);
+  keep.add(rest, n1 * 4);
+  keep.add(split, n1 * 4);
+  keep.add(h.own, kOwnWords * 4);
+  DevBuf mem, tmp_mem;  // mem becomes h.mem when it is complete
+  DevView rowbase, chunks, flag, pos, meta, cost, prefix, total, scan;
+  const size_t sb = tc_hub_scan_bytes(n, runs);
+  if (sb == 0) return fail(MGPM_ERR_HIP, "scan size query");
+  DevArena work;
+  for (DevView *v : {&rowbase, &chunks, &flag, &pos}) work.add(*v, n1 * 4);
+  work.add(meta, n1 * 16);
+  work.add(cost, (size_t(runs) + 1) * 8);
+  work.add(prefix, (size_t(runs) + 1) * 8);
+  work.add(total, 4);
+  work.add(scan, sb);
+  MGPM_HIP(keep.alloc(mem));
+  MGPM_HIP(work.alloc(tmp_mem));
+  p.rows = rows.p;
   p.owner = owner.as<HubOwner>();
   p.part = part.as<HubPartner>();
-  if (p.blocks &&
-      tc_hub_blocks(p, runs, cost.as<unsigned long long>(),
-                    prefix.as<unsigned long long>(), tmp.p, sb,
-                    bound.as<uint32_t>(), start.as<uint32_t>(), s))
-    return fail(MGPM_ERR_HIP, "hub plan kernel launch failed");
-  MGPM_HIP(hipStreamSynchronize(s));  // the work arrays die here
-  p.rows = rows.p;
   p.bound = bound.as<uint32_t>();
   p.start = start.as<uint32_t>();
   p.rest = rest.as<int32_t>();
   p.drp = drp;
   p.dcol = dcol;
   p.split = split.as<uint32_t>();
-  h.split.swap(split);
-  h.rows.swap(rows);
-  h.owner.swap(owner);
-  h.part.swap(part);
-  h.bound.swap(bound);
-  h.start.swap(start);
-  h.rest.swap(rest);
-  h.own.swap(own);
+  const uint32_t *owners = pos.as<uint32_t>() + n;
+  if (tc_hub_counts(drp, dcol, n, hublo, split.as<uint32_t>(),
+                    chunks.as<uint32_t>(), s) ||
+      tc_hub_scan(chunks.as<uint32_t>(), rowbase.as<uint32_t>(), n, scan.p,
+                  sb, s) ||
+      device_zero(total.p, 1, s) || device_zero(h.own.p, kOwnWords, s) ||
+      tc_hub_fill(cg.rowptr.as<int64_t>(), cg.col.as<int32_t>(),
+                  cg.src.as<int32_t>(), nnz, drp, dcol, cg.arc.as<uint32_t>(),
+                  n, split.as<uint32_t>(), rowbase.as<uint32_t>(), rows.p,
+                  flag.as<uint32_t>(), pos.as<uint32_t>(), meta.p,
+                  owner.as<HubOwner>(), part.as<HubPartner>(),
+                  rest.as<int32_t>(), total.as<uint32_t>(), scan.p, sb,
+                  dg->cus, s) ||
+      tc_hub_blocks(p, owners, runs, cost.as<unsigned long long>(),
+                    prefix.as<unsigned long long>(), scan.p, sb,
+                    bound.as<uint32_t>(), start.as<uint32_t>(), s))
+    return fail(MGPM_ERR_HIP, "hub plan kernel launch failed");
+  MGPM_HIP(hipMemcpyAsync(&p.nrest, total.p, 4, hipMemcpyDeviceToHost, s));
+  MGPM_HIP(hipMemcpyAsync(&p.owners, owners, 4, hipMemcpyDeviceToHost, s));
+  MGPM_HIP(hipStreamSynchronize(s));  // the work arrays die here
+  if (p.owners == 0) p.blocks = 0;  // no arc follows another: no triangle
+  h.mem.swap(mem);
   h.plan = p;
   h.ready = true;
   return MGPM_OK;

@@ -471,25 +471,36 @@ __global__ void hub_owner_list(const int64_t *__restrict__ rowptr,
       owner[pos[b]] = owner_of(rowptr, drp, rowbase, b);
 }
 
+// What a partner record needs of its row's vertex, in one 16-byte load.
+__global__ void hub_meta(const int64_t *__restrict__ drp, int32_t n,
+                         const uint32_t *__restrict__ split,
+                         const uint32_t *__restrict__ rowbase,
+                         uint4 *__restrict__ meta) {
+  for (int64_t v = int64_t(blockIdx.x) * blockDim.x + threadIdx.x; v < n;
+       v += int64_t(gridDim.x) * blockDim.x) {
+    const uint32_t e = static_cast<uint32_t>(drp[v + 1]);
+    meta[v] = make_uint4(e, e - split[v], rowbase[v], 0u);
+  }
+}
+
 // One partner per CSR entry a below its row's vertex b: the chunks of a's
 // row that hold hubs past b (the heads past b are the last ones of N+(a)).
 __global__ void hub_partners(const int32_t *__restrict__ col,
                              const int32_t *__restrict__ src, int64_t nnz,
                              const int64_t *__restrict__ drp,
                              const uint32_t *__restrict__ arc,
-                             const uint32_t *__restrict__ split,
-                             const uint32_t *__restrict__ rowbase,
+                             const uint4 *__restrict__ meta,
                              HubPartner *__restrict__ part) {
   for (int64_t j = int64_t(blockIdx.x) * blockDim.x + threadIdx.x; j < nnz;
        j += int64_t(gridDim.x) * blockDim.x) {
     const int32_t b = src[j], a = col[j];
     if (a > b) continue;
-    const uint32_t e = static_cast<uint32_t>(drp[a + 1]);
-    const uint32_t past = e - 1u - arc[j], hubs = e - split[a];
-    HubPartner r;
-    r.base = rowbase[a];
-    r.chunks = (min(past, hubs) + kHubChunk - 1) / kHubChunk;
-    part[j - drp[b]] = r;
+    const uint4 r = meta[a];  // end of N+(a), its hubs, its row
+    const uint32_t past = r.x - 1u - arc[j];
+    HubPartner h;
+    h.base = r.z;
+    h.chunks = (min(past, r.y) + kHubChunk - 1) / kHubChunk;
+    part[j - drp[b]] = h;
   }
 }
 
@@ -498,18 +509,24 @@ __global__ void hub_partners(const int32_t *__restrict__ col,
 __global__ void hub_costs(const HubPartner *__restrict__ part,
                           uint32_t nparts, uint32_t runs,
                           u64 *__restrict__ cost) {
-  for (uint32_t r = blockIdx.x * blockDim.x + threadIdx.x; r <= runs;
-       r += gridDim.x * blockDim.x) {
-    u64 c = 0;
-    for (uint32_t i = r * kHubRun; i < min((r + 1) * kHubRun, nparts); ++i)
-      c += max(1u, (part[i].chunks + kLanes - 1u) / kLanes);
-    cost[r] = c;
+  static_assert(kHubRun == 16, "a run per 16 lanes");
+  const uint32_t gl = threadIdx.x % kHubRun;
+  for (uint32_t r = (blockIdx.x * blockDim.x + threadIdx.x) / kHubRun;
+       r <= runs; r += gridDim.x * blockDim.x / kHubRun) {
+    const uint32_t i = r * kHubRun + gl;
+    int c = 0;
+    if (r < runs && i < nparts)
+      c = static_cast<int>(max(1u, (part[i].chunks + kLanes - 1u) / kLanes));
+#pragma unroll
+    for (int d = 8; d >= 1; d >>= 1) c += __shfl_xor(c, d, 16);
+    if (gl == 0) cost[r] = static_cast<u64>(c);
   }
 }
 
 __global__ void hub_owner_costs(const HubOwner *__restrict__ owner,
-                                uint32_t owners, u64 *__restrict__ cost) {
-  for (uint32_t k = blockIdx.x * blockDim.x + threadIdx.x; k < owners;
+                                const uint32_t *__restrict__ owners,
+                                u64 *__restrict__ cost) {
+  for (uint32_t k = blockIdx.x * blockDim.x + threadIdx.x; k < *owners;
        k += gridDim.x * blockDim.x)
     atomicAdd(&cost[owner[k].beg / kHubRun], kOwnerCost);
 }
@@ -518,7 +535,8 @@ __global__ void hub_owner_costs(const HubOwner *__restrict__ owner,
 // the total.
 __global__ void hub_blocks(const u64 *__restrict__ prefix, uint32_t runs,
                            const HubOwner *__restrict__ owner,
-                           uint32_t owners, uint32_t nparts, uint32_t blocks,
+                           const uint32_t *__restrict__ owners,
+                           uint32_t nparts, uint32_t blocks,
                            uint32_t *__restrict__ bound,
                            uint32_t *__restrict__ start) {
   const u64 total = prefix[runs];
@@ -534,7 +552,7 @@ __global__ void hub_blocks(const u64 *__restrict__ prefix, uint32_t runs,
     const uint32_t at = g == blocks ? nparts : min(a * kHubRun, nparts);
     bound[g] = at;
     if (g == blocks) continue;
-    uint32_t lo = 0, hi = owners;  // first owner with end > at
+    uint32_t lo = 0, hi = *owners;  // first owner with end > at
     while (lo < hi) {
       const uint32_t mid = lo + (hi - lo) / 2;
       if (owner[mid].end <= at) lo = mid + 1;
@@ -544,23 +562,26 @@ __global__ void hub_blocks(const u64 *__restrict__ prefix, uint32_t runs,
   }
 }
 
-// Vertices with two or more heads below the hubs.
-__global__ void hub_rest_list(const int64_t *__restrict__ drp,
-                              const uint32_t *__restrict__ split, int32_t n,
-                              int32_t *__restrict__ rest,
-                              uint32_t *__restrict__ nrest) {
-  const int64_t stride = int64_t(gridDim.x) * blockDim.x;
-  for (int64_t v0 = int64_t(blockIdx.x) * blockDim.x; v0 < n; v0 += stride) {
-    const int64_t v = v0 + threadIdx.x;
-    const bool in = v < n && static_cast<int64_t>(split[v]) - drp[v] >= 2;
-    const u64 m = __ballot(in);
-    if (!m) continue;
-    uint32_t base = 0;
-    if (lane64() == 0)
-      base = atomicAdd(nrest, static_cast<uint32_t>(__popcll(m)));
-    base = __shfl(base, 0, 64);
-    if (in) rest[base + bits_below(m)] = static_cast<int32_t>(v);
+// Vertices with two or more heads below the hubs, one atomic per 1024.
+constexpr int kRestT = 1024;
+__global__ __launch_bounds__(kRestT) void hub_rest_list(
+    const int64_t *__restrict__ drp, const uint32_t *__restrict__ split,
+    int32_t n, int32_t *__restrict__ rest, uint32_t *__restrict__ nrest) {
+  __shared__ uint32_t s_wave[kRestT / 64];
+  __shared__ uint32_t s_base;
+  const int64_t v = int64_t(blockIdx.x) * kRestT + threadIdx.x;
+  const bool in = v < n && static_cast<int64_t>(split[v]) - drp[v] >= 2;
+  const u64 m = __ballot(in);
+  if (lane64() == 0) s_wave[threadIdx.x >> 6] = __popcll(m);
+  __syncthreads();
+  uint32_t before = bits_below(m), total = 0;
+  for (int w = 0; w < kRestT / 64; ++w) {
+    if (w < static_cast<int>(threadIdx.x >> 6)) before += s_wave[w];
+    total += s_wave[w];
   }
+  if (threadIdx.x == 0) s_base = total ? atomicAdd(nrest, total) : 0u;
+  __syncthreads();
+  if (in) rest[s_base + before] = static_cast<int32_t>(v);
 }
 
 int flat(int64_t items, int most) {
@@ -616,18 +637,20 @@ int tc_hub_scan(const uint32_t *chunks, uint32_t *rowbase, int32_t n,
              : -1;
 }
 
-int tc_hub_blocks(const TcHubPlan &p, uint32_t runs, unsigned long long *cost,
-                  unsigned long long *prefix, void *tmp, size_t bytes,
-                  uint32_t *bound, uint32_t *start, hipStream_t s) {
-  hipLaunchKernelGGL(hub_costs, dim3(flat(int64_t(runs) + 1, 4096)),
+int tc_hub_blocks(const TcHubPlan &p, const uint32_t *owners, uint32_t runs,
+                  unsigned long long *cost, unsigned long long *prefix,
+                  void *tmp, size_t bytes, uint32_t *bound, uint32_t *start,
+                  hipStream_t s) {
+  hipLaunchKernelGGL(hub_costs, dim3(flat((int64_t(runs) + 1) * kHubRun,
+                                          8192)),
                      dim3(256), 0, s, p.part, p.nparts, runs, cost);
-  hipLaunchKernelGGL(hub_owner_costs, dim3(flat(p.owners, 4096)), dim3(256),
-                     0, s, p.owner, p.owners, cost);
+  hipLaunchKernelGGL(hub_owner_costs, dim3(flat(p.n, 4096)), dim3(256), 0, s,
+                     p.owner, owners, cost);
   if (hipcub::DeviceScan::ExclusiveSum(tmp, bytes, cost, prefix,
                                        int64_t(runs) + 1, s) != hipSuccess)
     return -1;
   hipLaunchKernelGGL(hub_blocks, dim3(flat(int64_t(p.blocks) + 1, 4096)),
-                     dim3(256), 0, s, prefix, runs, p.owner, p.owners,
+                     dim3(256), 0, s, prefix, runs, p.owner, owners,
                      p.nparts, p.blocks, bound, start);
   return hipGetLastError() == hipSuccess ? 0 : -1;
 }
@@ -636,7 +659,7 @@ int tc_hub_fill(const int64_t *rowptr, const int32_t *col,
                 const int32_t *src, int64_t nnz, const int64_t *drp,
                 const int32_t *dcol, const uint32_t *arc, int32_t n,
                 const uint32_t *split, uint32_t *rowbase, void *rows,
-                uint32_t *flag, uint32_t *pos, HubOwner *owner,
+                uint32_t *flag, uint32_t *pos, void *meta, HubOwner *owner,
                 HubPartner *part, int32_t *rest, uint32_t *nrest, void *tmp,
                 size_t bytes, int cus, hipStream_t s) {
   hipLaunchKernelGGL(hub_rows, dim3(flat(int64_t(n) * 64, cus * 32)),
@@ -648,10 +671,13 @@ int tc_hub_fill(const int64_t *rowptr, const int32_t *col,
   if (tc_hub_scan(flag, pos, n, tmp, bytes, s)) return -1;
   hipLaunchKernelGGL(hub_owner_list, dim3(flat(n, 4096)), dim3(256), 0, s,
                      rowptr, drp, rowbase, n, pos, owner);
+  hipLaunchKernelGGL(hub_meta, dim3(flat(n, 4096)), dim3(256), 0, s, drp, n,
+                     split, rowbase, static_cast<uint4 *>(meta));
   hipLaunchKernelGGL(hub_partners, dim3(flat(nnz, cus * 32)), dim3(256), 0, s,
-                     col, src, nnz, drp, arc, split, rowbase, part);
-  hipLaunchKernelGGL(hub_rest_list, dim3(flat(n, 1024)), dim3(256), 0, s, drp,
-                     split, n, rest, nrest);
+                     col, src, nnz, drp, arc,
+                     static_cast<const uint4 *>(meta), part);
+  hipLaunchKernelGGL(hub_rest_list, dim3(n / kRestT + 1), dim3(kRestT), 0, s,
+                     drp, split, n, rest, nrest);
   return hipGetLastError() == hipSuccess ? 0 : -1;
 }
 

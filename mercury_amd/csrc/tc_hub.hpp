@@ -67,7 +67,8 @@ int tc_hub_launch(const TcHubPlan &p, const HubOut &out, int cus,
 
 // Preparation: split (n) and the chunks of every row (n + 1, the last 0);
 // the caller scans them into rowbase, then the rows, owners (flag and pos
-// hold n + 1 entries, pos[n] their number), partners and the rest list
+// hold n + 1 entries, pos[n] their number; meta 16 bytes per vertex),
+// partners and the rest list
 // (its size into *nrest, zeroed), then the blocks (runs = ceil(nparts /
 // kHubRun); cost and prefix hold runs + 1 entries).
 int tc_hub_counts(const int64_t *drp, const int32_t *dcol, int32_t n,
@@ -80,11 +81,12 @@ int tc_hub_fill(const int64_t *rowptr, const int32_t *col,
                 const int32_t *src, int64_t nnz, const int64_t *drp,
                 const int32_t *dcol, const uint32_t *arc, int32_t n,
                 const uint32_t *split, uint32_t *rowbase, void *rows,
-                uint32_t *flag, uint32_t *pos, HubOwner *owner,
+                uint32_t *flag, uint32_t *pos, void *meta, HubOwner *owner,
                 HubPartner *part, int32_t *rest, uint32_t *nrest, void *tmp,
                 size_t bytes, int cus, hipStream_t s);
-int tc_hub_blocks(const TcHubPlan &p, uint32_t runs, unsigned long long *cost,
-                  unsigned long long *prefix, void *tmp, size_t bytes,
-                  uint32_t *bound, uint32_t *start, hipStream_t s);
+int tc_hub_blocks(const TcHubPlan &p, const uint32_t *owners, uint32_t runs,
+                  unsigned long long *cost, unsigned long long *prefix,
+                  void *tmp, size_t bytes, uint32_t *bound, uint32_t *start,
+                  hipStream_t s);
 
 }  // namespace mgpm
