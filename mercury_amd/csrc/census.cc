@@ -235,6 +235,7 @@ CensusArgs args_of(mgpm_dgraph *dg, int passes, CensusWork &w,
   c.m = dg->host->nnz / 2;
   c.t = w.t.as<uint32_t>();
   c.arc = cg.arc.as<uint32_t>();
+  c.src = cg.src.as<int32_t>();
   c.order = cg.order.as<int32_t>();
   c.winlo = std::max<int32_t>(0, c.n - kRowWindow);
   c.cursor = cursor_of(w);
@@ -261,9 +262,7 @@ Census5Args args5_of(mgpm_dgraph *dg, CensusWork &w, const Need &k) {
   c.nnz = dg->host->nnz;
   c.drp = cg.drp.as<int64_t>();
   c.dcol = cg.dcol.as<int32_t>();
-  c.arc = cg.arc.as<uint32_t>();
   c.t = w.t.as<uint32_t>();
-  c.t_csr = w.t_csr.as<uint32_t>();
   c.tv = w.tv.as<unsigned long long>();
   c.anchors = w.anchors.as<int32_t>();
   char *sm = w.small.as<char>();

@@ -91,6 +91,7 @@ struct CensusArgs {
   const int64_t *rowptr = nullptr;
   const int32_t *col = nullptr;
   const uint32_t *arc = nullptr;
+  const int32_t *src = nullptr;  // row of every CSR entry
   // Vertices with out-neighbours, by class of their number (RowClass), and
   // the lowest id of the rows' bitmap window.
   const int32_t *order = nullptr;
@@ -102,10 +103,10 @@ struct CensusArgs {
   unsigned *c4_cursor = nullptr;
   uint32_t *wedges = nullptr;
   // 5-vertex census extras (P2, P3, P5, P6): the terms above marked full5
-  // are accumulated only when set; t_csr holds t_e per undirected CSR arc
-  // (census_t_csr) for the 4-cycle pass, tv twice the triangles per vertex.
+  // are accumulated only when set; t_csr gets t_e per CSR entry and tv twice
+  // the triangles per vertex (zeroed) from census_sums_launch.
   bool full5 = false;
-  const uint32_t *t_csr = nullptr;
+  uint32_t *t_csr = nullptr;
   unsigned long long *tv = nullptr;
 };
 
@@ -146,8 +147,6 @@ struct Census5Args {
   const int64_t *drp = nullptr;      // DAG
   const int32_t *dcol = nullptr;
   const uint32_t *t = nullptr;       // per DAG arc triangles
-  const uint32_t *arc = nullptr;     // DAG arc of every CSR entry (nnz)
-  uint32_t *t_csr = nullptr;         // out: per CSR arc triangles (nnz)
   const unsigned long long *tv = nullptr;  // twice the triangles per vertex
   // Anchor classes: ids grouped by class (n), class sizes and the starts
   // of the classes in `anchors` (kC5Classes each, zeroed before
@@ -178,8 +177,8 @@ struct Census5Args {
   unsigned long long *acc = nullptr; // kCensusSlots
 };
 
-// Enqueues t_csr and the per-vertex sums (kCensusTriS, kCensusTv2); needs
-// t and tv from the row pass and census_sums_launch.
+// Enqueues the per-vertex sums (kCensusTriS, kCensusTv2, kCensusCricket);
+// needs tv from census_sums_launch.
 int census5_flat_launch(const Census5Args &c, int cus, hipStream_t s);
 // Enqueues the pair-table count pass (tab_cap, from zeroed stamps); the
 // caller scans tab_cap into tab_off and sizes the table from tab_off[n].
@@ -220,7 +219,8 @@ int census_rows_launch(const CensusArgs &c, const int64_t *cls_count,
                        int64_t max_out, bool cliques, char *slab,
                        size_t budget, int cus, hipStream_t s);
 
-// Enqueues the sums over vertices and edges (needs t).
+// Enqueues the sums over vertices and edges (needs t), with full5 also t_csr
+// and tv.
 int census_sums_launch(const CensusArgs &c, int cus, hipStream_t s);
 
 // The 4-cycle pass's owners by kind (both ends in the window, the lower

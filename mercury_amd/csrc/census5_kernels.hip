@@ -113,16 +113,13 @@ __device__ __forceinline__ unsigned long long wg_sum(unsigned long long x,
   return t;
 }
 
-// t per undirected CSR arc, from its DAG arc.
-__global__ void c5_t_csr(Census5Args c) {
-  for (int64_t j = int64_t(blockIdx.x) * blockDim.x + threadIdx.x; j < c.nnz;
-       j += int64_t(gridDim.x) * blockDim.x)
-    c.t_csr[j] = c.t[c.arc[j]];
-}
-
 // Sums over vertices of C(t_v, 2) and t_v C(d_v - 2, 2), and of t_v s_v as
 // a sum over CSR arcs (v, x) of t_v (d_x - 1).
-__global__ void c5_flat(Census5Args c) {
+constexpr int kFlatT = 1024;
+__global__ __launch_bounds__(kFlatT) void c5_flat(Census5Args c) {
+  __shared__ unsigned long long s_sum[3];
+  if (threadIdx.x < 3) s_sum[threadIdx.x] = 0;
+  __syncthreads();
   unsigned long long ts = 0, t2 = 0, crk = 0;
   const int64_t stride = int64_t(gridDim.x) * blockDim.x;
   const int64_t i0 = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
@@ -139,9 +136,15 @@ __global__ void c5_flat(Census5Args c) {
   t2 = wave_sum_u64(t2);
   crk = wave_sum_u64(crk);
   if (lane64() == 0) {
-    if (crk) atomicAdd(&c.acc[kCensusCricket], crk);
-    if (ts) atomicAdd(&c.acc[kCensusTriS], ts);
-    if (t2) atomicAdd(&c.acc[kCensusTv2], t2);
+    atomicAdd(&s_sum[0], ts);
+    atomicAdd(&s_sum[1], t2);
+    atomicAdd(&s_sum[2], crk);
+  }
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    if (s_sum[0]) atomicAdd(&c.acc[kCensusTriS], s_sum[0]);
+    if (s_sum[1]) atomicAdd(&c.acc[kCensusTv2], s_sum[1]);
+    if (s_sum[2]) atomicAdd(&c.acc[kCensusCricket], s_sum[2]);
   }
 }
 
@@ -514,10 +517,10 @@ size_t census5_group_bytes(int32_t n, int words) {
 }
 
 int census5_flat_launch(const Census5Args &c, int cus, hipStream_t s) {
-  const int g = std::max(1, std::min(cus * 8, static_cast<int>(
-                                                  (c.nnz + 255) / 256)));
-  hipLaunchKernelGGL(c5_t_csr, dim3(g), dim3(256), 0, s, c);
-  hipLaunchKernelGGL(c5_flat, dim3(g), dim3(256), 0, s, c);
+  const int64_t items = std::max<int64_t>(c.n, c.nnz);
+  const int g = static_cast<int>(std::max<int64_t>(
+      1, std::min<int64_t>((items + kFlatT - 1) / kFlatT, int64_t(cus) * 2)));
+  hipLaunchKernelGGL(c5_flat, dim3(g), dim3(kFlatT), 0, s, c);
   return hipGetLastError() == hipSuccess ? 0 : -1;
 }
 
