@@ -532,7 +532,8 @@ int mgpm_dgraph_upload_ex(const mgpm_graph *g, int device, void *stream,
   if (rc) return rc;
   static bool inited = false;
   if (!inited) {
-    if (tc_device_init() || census_rows_init() || census_c4_init())
+    if (tc_device_init() || census_rows_init() || census_c4_init() ||
+        census5_init())
       return fail(MGPM_ERR_HIP, "kernel attribute setup");
     inited = true;
   }

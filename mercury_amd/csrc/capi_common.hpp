@@ -198,11 +198,16 @@ struct CensusGraph {
   bool c4_ready = false;
   DevBuf c4_win, c4_list;
   uint32_t c4_count[3][2] = {{0, 0}, {0, 0}, {0, 0}};
+  // Pair passes, likewise: pair-table slots and the n + 1 offsets of the
+  // anchors' parts, the anchors by list (sizes in c5_count), and every row's
+  // offsets of the fine windows.
   bool pairs_ready = false;
-  uint64_t tab_total = 0;  // pair-table slots
-  DevBuf tab_off;          // n + 1 slot offsets
+  uint64_t tab_total = 0;
+  DevBuf tab_off, c5_list, c5_woff;
+  uint32_t c5_count[6] = {0, 0, 0, 0, 0, 0};
   size_t bytes() const {
-    return mem.bytes + c4_win.bytes + c4_list.bytes + tab_off.bytes;
+    return mem.bytes + c4_win.bytes + c4_list.bytes + tab_off.bytes +
+           c5_list.bytes + c5_woff.bytes;
   }
 };
 
@@ -227,10 +232,10 @@ struct CensusWork {
   // batch lanes and server slots less.
   size_t budget = size_t(16) << 30;
   DevBuf t, t_csr, tv, small, slab, wedges;
-  DevBuf stamp, lo, mask, list, grows, anchors, table;
+  DevBuf lo, mask, list, grows, table;
   size_t bytes() const {
     return t.bytes + t_csr.bytes + tv.bytes + small.bytes + slab.bytes +
-           wedges.bytes + stamp.bytes + lo.bytes + mask.bytes + list.bytes + grows.bytes + anchors.bytes +
+           wedges.bytes + lo.bytes + mask.bytes + list.bytes + grows.bytes +
            table.bytes;
   }
 };

@@ -56,13 +56,11 @@ constexpr size_t kCensusC4Budget = size_t(4) << 30;
 constexpr size_t kCensusRowBudget = size_t(8) << 30;  // row passes' slabs
 constexpr size_t kCensus5Budget = size_t(8) << 30;  // pair-table layout
 
-// Layout of the small buffer: census cursors, accumulators, pair-pass
-// cursors and class counters.
+// Layout of the small buffer: census cursors, accumulators, pair-pass and
+// 4-cycle cursors.
 constexpr size_t kSmallBytes = 1024;
 constexpr size_t kAccOff = 64;
 constexpr size_t kC5CursorOff = 384;
-constexpr size_t kClsCountOff = 448;
-constexpr size_t kClsFillOff = 480;
 constexpr size_t kC4CursorOff = 512;
 
 // `passes` is a census_passes mask: the triangle pass and the sums always
@@ -93,9 +91,9 @@ int zero(void *p, size_t bytes, hipStream_t s) {
 // Sizes of the workspace for one pattern on one graph.
 struct Need {
   size_t t = 0, t_csr = 0, tv = 0, slab = 0, wedges = 0;
-  size_t stamp = 0, mask = 0, grows = 0, anchors = 0, table = 0;
-  int c4_groups = 0, groups = 0;
-  int64_t mask_words = 0, grows_len = 0;
+  size_t lo = 0, mask = 0, grows = 0, table = 0;
+  int c4_groups = 0, c5_groups[kC5Lists] = {};
+  int64_t grows_len = 0;
 };
 
 // Slab bytes of the row passes: the classes run one after the other on one
@@ -138,21 +136,25 @@ Need need_for(const mgpm_dgraph *dg, int passes, size_t budget) {
     k.t_csr = static_cast<size_t>(nnz);
     k.tv = static_cast<size_t>(n);
     const int gen_words = static_cast<int>((cg.max_out + 63) / 64);
-    // Half the budget to stamps, pending counts and lists (12 bytes per
-    // vertex per workgroup), half to masks: the one- and two-word classes
-    // (nearly every anchor) get every workgroup, wider classes fewer.
-    const size_t half = budget / 2;
-    k.groups = static_cast<int>(std::max<size_t>(
-        1, std::min<size_t>({size_t(dg->cus) * 4, size_t(n),
-                             half / (12 * size_t(n))})));
-    const int64_t wmax = std::max<int64_t>(8, gen_words);
-    k.mask_words = std::min<int64_t>(half / (8 * size_t(n)), 2 * k.groups);
-    k.mask_words = std::max<int64_t>(k.mask_words, wmax);
-    k.stamp = static_cast<size_t>(k.groups) * n;
-    k.mask = static_cast<size_t>(k.mask_words) * n;
+    // Half the budget per list of anchors: the lists run one after the
+    // other on arrays as large as the largest of each kind (before the plan
+    // is built: as if every list held all vertices).
+    const int32_t winlo = std::max<int32_t>(0, G.n - kRowWindow);
+    for (int q = 0; q < kC5Lists; ++q) {
+      const bool gen = q == kC5Lists - 1;
+      int64_t count = cg.pairs_ready ? cg.c5_count[q] : n;
+      if (gen && gen_words <= kC5Words[kC5Windowed - 1]) count = 0;
+      const int g = census5_groups(q, count, G.n, winlo, gen_words,
+                                   budget / 2, dg->cus);
+      k.c5_groups[q] = g;
+      if (!g) continue;
+      const size_t range = size_t(g) * size_t(gen ? n : winlo);
+      const size_t words = size_t(gen ? gen_words : kC5Words[q - 1]);
+      k.lo = std::max(k.lo, range);
+      k.mask = std::max(k.mask, range * words);
+      if (gen) k.grows = size_t(g) * cg.max_out * gen_words;
+    }
     k.grows_len = cg.max_out * gen_words;
-    k.grows = static_cast<size_t>(k.groups) * k.grows_len;
-    k.anchors = static_cast<size_t>(n);
     k.table = cg.tab_total;
   }
   return k;
@@ -264,22 +266,22 @@ Census5Args args5_of(mgpm_dgraph *dg, CensusWork &w, const Need &k) {
   c.dcol = cg.dcol.as<int32_t>();
   c.t = w.t.as<uint32_t>();
   c.tv = w.tv.as<unsigned long long>();
-  c.anchors = w.anchors.as<int32_t>();
-  char *sm = w.small.as<char>();
-  c.cls_count = reinterpret_cast<unsigned *>(sm + kClsCountOff);
-  c.cls_fill = reinterpret_cast<unsigned *>(sm + kClsFillOff);
-  c.stamp = w.stamp.as<uint32_t>();
+  c.arc = cg.arc.as<uint32_t>();
+  c.anchors = cg.c5_list.as<int32_t>();
+  c.winlo = std::max<int32_t>(0, c.n - kRowWindow);
+  c.nf = census5_fine_windows(c.n, c.winlo);
+  c.win = cg.c4_win.as<uint32_t>();
+  c.woff = cg.c5_woff.as<uint16_t>();
   c.lo = w.lo.as<uint32_t>();
   c.mask = w.mask.as<unsigned long long>();
   c.list = w.list.as<int32_t>();
-  c.groups = k.groups;
-  c.mask_words = k.mask_words;
   c.gen_words = static_cast<int>((cg.max_out + 63) / 64);
   c.grows = w.grows.as<unsigned long long>();
   c.grows_len = k.grows_len;
   c.tab_off = cg.tab_off.as<unsigned long long>();
   c.table = w.table.as<unsigned long long>();
-  c.cursor = reinterpret_cast<unsigned *>(sm + kC5CursorOff);
+  c.cursor =
+      reinterpret_cast<unsigned *>(w.small.as<char>() + kC5CursorOff);
   c.acc = census_acc(w);
   return c;
 }
@@ -302,11 +304,9 @@ int work_grow(CensusWork &w, const Need &k, hipStream_t s) {
   if (k.t_csr) {
     if ((rc = grow<uint32_t>(w.t_csr, k.t_csr))) return rc;
     if ((rc = grow<unsigned long long>(w.tv, k.tv))) return rc;
-    if ((rc = grow<int32_t>(w.anchors, k.anchors))) return rc;
     if ((rc = grow<unsigned long long>(w.table, k.table))) return rc;
-    if ((rc = grow<uint32_t>(w.stamp, k.stamp))) return rc;
-    if ((rc = grow<int32_t>(w.list, k.stamp))) return rc;
-    if ((rc = grow_z(w.lo, k.stamp * 4))) return rc;
+    if ((rc = grow<int32_t>(w.list, k.lo))) return rc;
+    if ((rc = grow_z(w.lo, k.lo * 4))) return rc;
     if ((rc = grow_z(w.mask, k.mask * 8))) return rc;
     if ((rc = grow<unsigned long long>(w.grows, k.grows))) return rc;
   }
@@ -333,8 +333,8 @@ uint64_t census_work_bytes(const mgpm_dgraph *dg, int passes,
   }
   const Need k = need_for(dg, passes, budget);
   return 4ull * k.t + kSmallBytes + k.slab + 4ull * k.wedges +
-         4ull * k.t_csr + 8ull * k.tv + 12ull * k.stamp +
-         8ull * k.mask + 8ull * k.grows + 4ull * k.anchors + 8ull * k.table;
+         4ull * k.t_csr + 8ull * k.tv + 8ull * k.lo + 8ull * k.mask +
+         8ull * k.grows + 8ull * k.table;
 }
 
 namespace {
@@ -394,54 +394,90 @@ int c4_layout(mgpm_dgraph *dg, hipStream_t s) {
   return MGPM_OK;
 }
 
-// The pair-table layout of the graph (once): per anchor, a power of two of
-// slots at least twice the pairs it will hold, from one count pass over
-// temporary stamps, one scan and one read of the total.
+// The pair passes' plan of the graph (once): per anchor, a power of two of
+// table slots at least twice the pairs it will hold, from one count pass
+// over temporary stamps and one scan; the anchors by list; the offsets of
+// the fine windows in every row.  Two reads: list sizes, table slots.
 int pairs_layout(mgpm_dgraph *dg, hipStream_t s) {
   CensusGraph &cg = dg->census;
   if (cg.pairs_ready) return MGPM_OK;
   const int32_t n = dg->host->n;
   const int64_t nnz = dg->host->nnz;
-  const size_t n1 = static_cast<size_t>(n) + 1;
-  const int groups = static_cast<int>(std::max<size_t>(
-      1, std::min<size_t>(size_t(dg->cus) * 2,
-                          (kCensus5Budget / 4) /
-                              (4 * std::max<size_t>(n, 1)))));
-  DevBuf off, cap, stamp, small, scan;
-  size_t sb = 0;
-  if (census5_scan_bytes(int64_t(n1), &sb))
-    return fail(MGPM_ERR_HIP, "scan size query");
-  MGPM_HIP(off.alloc(n1 * 8));
-  MGPM_HIP(cap.alloc(n1 * 8));
-  MGPM_HIP(stamp.alloc(size_t(groups) * std::max<size_t>(n, 1) * 4));
-  MGPM_HIP(small.alloc(kSmallBytes));
-  MGPM_HIP(scan.alloc(std::max<size_t>(sb, 1)));
+  const size_t n0 = std::max<size_t>(n, 1), n1 = static_cast<size_t>(n) + 1;
   Census5Args c;
   c.rowptr = cg.rowptr.as<int64_t>();
   c.col = cg.col.as<int32_t>();
+  c.src = cg.src.as<int32_t>();
   c.deg = cg.deg.as<int32_t>();
   c.n = n;
   c.nnz = nnz;
   c.drp = cg.drp.as<int64_t>();
   c.dcol = cg.dcol.as<int32_t>();
+  c.arc = cg.arc.as<uint32_t>();
+  c.winlo = std::max<int32_t>(0, n - kRowWindow);
+  c.nf = census5_fine_windows(n, c.winlo);
+  c.win = cg.c4_win.as<uint32_t>();
+  const size_t below = std::max<size_t>(c.winlo, 1);
+  c.groups = static_cast<int>(std::max<size_t>(
+      1, std::min<size_t>(size_t(dg->cus) * 2,
+                          (kCensus5Budget / 4) / (4 * below))));
+  constexpr size_t kCls = 3 * kC5Lists * sizeof(unsigned);
+  size_t sb = 0;
+  if (census5_scan_bytes(int64_t(n1), &sb))
+    return fail(MGPM_ERR_HIP, "scan size query");
+  DevBuf off, list, woff, mem;
+  DevArena work;
+  DevView cap, stamp, small, scan, cls, cnt;  // cnt: sizes, starts, fills
+  work.add(cap, n1 * 8);
+  work.add(stamp, size_t(c.groups) * below * 4);
+  work.add(small, kSmallBytes);
+  work.add(scan, std::max<size_t>(sb, 1));
+  work.add(cls, n0);
+  work.add(cnt, kCls);
+  MGPM_HIP(off.alloc(n1 * 8));
+  MGPM_HIP(woff.alloc(n0 * (c.nf + 1) * sizeof(uint16_t)));
+  MGPM_HIP(work.alloc(mem));
   c.stamp = stamp.as<uint32_t>();
-  c.groups = groups;
   c.tab_cap = cap.as<unsigned long long>();
   c.cursor = reinterpret_cast<unsigned *>(small.as<char>() + kC5CursorOff);
+  unsigned *sizes_d = cnt.as<unsigned>();
   int rc;
   if ((rc = zero(small.p, kSmallBytes, s))) return rc;
-  if ((rc = zero(stamp.p, stamp.bytes, s))) return rc;
+  if (c.winlo && (rc = zero(stamp.p, size_t(c.groups) * below * 4, s)))
+    return rc;
   if ((rc = zero(cap.p, n1 * 8, s))) return rc;
-  if (census5_table_count_launch(c, s))
+  if ((rc = zero(cnt.p, kCls, s))) return rc;
+  if (census5_classes(c, cls.as<int8_t>(), sizes_d, s) ||
+      census5_window_offsets(c, woff.as<uint16_t>(), dg->cus, s))
+    return fail(MGPM_ERR_HIP, "census kernel launch failed");
+  unsigned sizes[kC5Lists], starts[kC5Lists];
+  MGPM_HIP(hipMemcpyAsync(sizes, sizes_d, sizeof(sizes),
+                          hipMemcpyDeviceToHost, s));
+  MGPM_HIP(hipStreamSynchronize(s));
+  size_t at = 0;
+  for (int k = 0; k < kC5Lists; ++k) {
+    starts[k] = static_cast<unsigned>(at);
+    at += sizes[k];
+  }
+  MGPM_HIP(list.alloc(std::max<size_t>(at, 1) * sizeof(int32_t)));
+  c.anchors = list.as<int32_t>();
+  MGPM_HIP(hipMemcpyAsync(sizes_d + kC5Lists, starts, sizeof(starts),
+                          hipMemcpyHostToDevice, s));
+  if (census5_lists(n, cls.as<int8_t>(), sizes_d + kC5Lists,
+                    sizes_d + 2 * kC5Lists, list.as<int32_t>(), s) ||
+      census5_table_count_launch(c, sizes, dg->cus, s))
     return fail(MGPM_ERR_HIP, "census kernel launch failed");
   if (census5_scan(cap.as<unsigned long long>(), off.as<unsigned long long>(),
-                   int64_t(n1), scan.p, scan.bytes, s))
+                   int64_t(n1), scan.p, sb, s))
     return fail(MGPM_ERR_HIP, "census scan failed");
   unsigned long long total = 0;
   MGPM_HIP(hipMemcpyAsync(&total, off.as<unsigned long long>() + n, 8,
                           hipMemcpyDeviceToHost, s));
-  MGPM_HIP(hipStreamSynchronize(s));
+  MGPM_HIP(hipStreamSynchronize(s));  // the work arrays die here
+  for (int k = 0; k < kC5Lists; ++k) cg.c5_count[k] = sizes[k];
   cg.tab_off.swap(off);
+  cg.c5_list.swap(list);
+  cg.c5_woff.swap(woff);
   cg.tab_total = total;
   cg.pairs_ready = true;
   return MGPM_OK;
@@ -507,10 +543,7 @@ int census_enqueue(mgpm_dgraph *dg, int passes, CensusWork &w,
     return fail(MGPM_ERR_HIP, "census kernel launch failed");
   if (f5) {
     if ((rc = zero(w.table.p, cg.tab_total * 8, s))) return rc;
-    if (census5_classify_launch(c5, s))
-      return fail(MGPM_ERR_HIP, "census kernel launch failed");
-    if ((rc = zero(w.stamp.p, w.stamp.bytes, s))) return rc;
-    if (census5_pairs_launch(c5, s))
+    if (census5_pairs_launch(c5, cg.c5_count, k.c5_groups, dg->cus, s))
       return fail(MGPM_ERR_HIP, "census kernel launch failed");
   }
   return MGPM_OK;

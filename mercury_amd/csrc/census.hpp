@@ -130,12 +130,23 @@ struct RowArgs {
 
 // The pair passes of the 5-vertex census (census5_kernels.hip).  Anchors
 // are the vertices, each processed as the lowest-ranked vertex (DAG order:
-// degree, then id) of the occurrences it accounts for, in classes by DAG
-// out-degree d+ (kC5Classes; class k < kC5Classes - 1 holds d+ up to
-// 64 * kC5Words[k] and keeps the adjacency inside N+(a) in LDS, the last
-// class the rest, with it in a per-workgroup global slab).
-constexpr int kC5Classes = 5;
-constexpr int kC5Words[kC5Classes - 1] = {1, 2, 4, 8};
+// degree, then id) of the occurrences it accounts for, in lists: light ones
+// (few items), then by DAG out-degree d+ up to 64 * kC5Words[k] with the
+// targets of the window in LDS, then the rest with everything in global
+// memory.
+constexpr int kC5Windowed = 4;
+constexpr int kC5Words[kC5Windowed] = {1, 2, 4, 8};
+constexpr int kC5Light = 0;                  // list of the light anchors
+constexpr int kC5Lists = kC5Windowed + 2;
+constexpr unsigned kLightItems = 256;
+constexpr int kFine = 1664;                  // ids of a fine window
+
+struct C5List {
+  const int32_t *list = nullptr;
+  uint32_t count = 0;
+  uint32_t grab = 1;  // per queue access
+  unsigned *cursor = nullptr;
+};
 
 struct Census5Args {
   const int64_t *rowptr = nullptr;   // undirected CSR
@@ -148,23 +159,23 @@ struct Census5Args {
   const int32_t *dcol = nullptr;
   const uint32_t *t = nullptr;       // per DAG arc triangles
   const unsigned long long *tv = nullptr;  // twice the triangles per vertex
-  // Anchor classes: ids grouped by class (n), class sizes and the starts
-  // of the classes in `anchors` (kC5Classes each, zeroed before
-  // classification).
-  int32_t *anchors = nullptr;
-  unsigned *cls_count = nullptr;
-  unsigned *cls_fill = nullptr;
-  // Per-workgroup dense arrays over all vertices: stamps (n u32, zeroed
-  // once), pending counts lo (n u32) and masks (n x words u64) (zeroed,
-  // and left zeroed), and a list of the vertices touched (n int32).
+  const uint32_t *arc = nullptr;     // DAG arc of every CSR entry
+  const int32_t *anchors = nullptr;  // the lists of anchors, in order
+  // The window: its lowest id, the first entry of every row in it, and per
+  // row the entries before each of nf fine windows (nf + 1 per row).
+  int32_t winlo = 0;
+  int nf = 0;
+  const uint32_t *win = nullptr;
+  const uint16_t *woff = nullptr;
+  // Per workgroup, for the targets below the window (or, last list, all):
+  // counts (u32) and masks (words x u64), zero and left zero, and a list of
+  // the targets touched; stamps of the count pass.
   uint32_t *stamp = nullptr;
   uint32_t *lo = nullptr;
   unsigned long long *mask = nullptr;
   int32_t *list = nullptr;
-  int groups = 0;                    // workgroups stamp/lo/list hold
-  int64_t mask_words = 0;            // mask buffer length / n (>= words of
-                                     // every class)
-  int gen_words = 1;                 // words per mask of the last class
+  int groups = 0;                    // workgroups of the count pass
+  int gen_words = 1;                 // words per mask of the last list
   unsigned long long *grows = nullptr;  // last class: rows per workgroup
   int64_t grows_len = 0;             // max d+ x gen_words
   // Pair table: codeg(p, q) of every pair (p below q) with a common
@@ -173,7 +184,7 @@ struct Census5Args {
   unsigned long long *tab_cap = nullptr;  // n + 1 (out of the count pass)
   unsigned long long *tab_off = nullptr;  // n + 1 (exclusive scan of cap)
   unsigned long long *table = nullptr;    // zeroed
-  unsigned *cursor = nullptr;        // 16 counters (zeroed)
+  unsigned *cursor = nullptr;        // 16 queue counters (zeroed)
   unsigned long long *acc = nullptr; // kCensusSlots
 };
 
@@ -182,18 +193,33 @@ struct Census5Args {
 int census5_flat_launch(const Census5Args &c, int cus, hipStream_t s);
 // Enqueues the pair-table count pass (tab_cap, from zeroed stamps); the
 // caller scans tab_cap into tab_off and sizes the table from tab_off[n].
-int census5_table_count_launch(const Census5Args &c, hipStream_t s);
-// Enqueues the classification of the anchors (cls_count, cls_fill zeroed).
-int census5_classify_launch(const Census5Args &c, hipStream_t s);
+int census5_table_count_launch(const Census5Args &c, const uint32_t *count,
+                               int cus, hipStream_t s);
+// The anchors' lists: classes of all vertices (n; list sizes into fill,
+// kC5Lists entries, zeroed), then, with fill zeroed again and the starts of
+// the lists, the lists.
+int census5_classes(const Census5Args &c, int8_t *cls, unsigned *fill,
+                    hipStream_t s);
+int census5_lists(int32_t n, const int8_t *cls, const unsigned *start,
+                  unsigned *fill, int32_t *list, hipStream_t s);
+// Fine windows of a graph, and the offsets of every row (n x (nf + 1)).
+int census5_fine_windows(int32_t n, int32_t winlo);
+int census5_window_offsets(const Census5Args &c, uint16_t *woff, int cus,
+                           hipStream_t s);
+// Raises the dynamic-LDS limits (once per process).
+int census5_init();
+// Workgroups of list `cls` whose global arrays fit `budget` bytes.
+int census5_groups(int cls, int64_t count, int32_t n, int32_t winlo,
+                   int gen_words, size_t budget, int cus);
 // Exclusive prefix sum of `count` uint64 values; tmp of census5_scan_bytes.
 int census5_scan_bytes(int64_t count, size_t *bytes);
 int census5_scan(const unsigned long long *in, unsigned long long *out,
                  int64_t count, void *tmp, size_t tmp_bytes, hipStream_t s);
-// Enqueues the anchor and out-neighbourhood passes of every class
-// (kCensusW4, kCensusK23, kCensusK23e, kCensusTableMiss).
-int census5_pairs_launch(const Census5Args &c, hipStream_t s);
-// Per-workgroup bytes of the dense arrays with masks of `words` words.
-size_t census5_group_bytes(int32_t n, int words);
+// Enqueues the anchor and out-neighbourhood passes of every list (sizes
+// count, workgroups groups; kCensusW4, kCensusK23, kCensusK23e,
+// kCensusTableMiss).
+int census5_pairs_launch(const Census5Args &c, const uint32_t *count,
+                         const int *groups, int cus, hipStream_t s);
 
 // Raises the dynamic-LDS limit of the row kernels (once per process).
 int census_rows_init();
