@@ -209,7 +209,7 @@ int graph_ready(mgpm_dgraph *dg, hipStream_t s) {
   int rc = zero(cls.p, kCls, s);
   if (rc) return rc;
   unsigned *cnt = cls.as<unsigned>();
-  if (census_rows_classify(c.drp, n, cnt, cnt + kRowClassCount,
+  if (census_rows_classify(c.drp, c.deg, n, cnt, cnt + kRowClassCount,
                            cg.order.as<int32_t>(), s))
     return fail(MGPM_ERR_HIP, "census kernel launch failed");
   unsigned sizes[kRowClassCount];

@@ -233,8 +233,9 @@ int rows_grid(int cls, int64_t max_out, int64_t count, bool cliques,
 
 // Enqueues the vertices by class into list (n entries), the class sizes
 // into count (kRowClassCount, with fill zeroed before the call).
-int census_rows_classify(const int64_t *drp, int32_t n, unsigned *count,
-                         unsigned *fill, int32_t *list, hipStream_t s);
+int census_rows_classify(const int64_t *drp, const int32_t *deg, int32_t n,
+                         unsigned *count, unsigned *fill, int32_t *list,
+                         hipStream_t s);
 
 // Enqueues one row pass over every class.  cliques = false: t of every arc
 // and kCensusK4; cliques = true (t complete): the per-triangle 4-clique

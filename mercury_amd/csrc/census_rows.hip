@@ -29,9 +29,11 @@
 // row intersections are LDS reads.  RMAT-20 (16 draws per vertex) streams
 // 4.4e9 + 1.2e9 items and intersects 9.6e9 word pairs.  Measured on one
 // MI355X against one wave per DAG arc with binary searches (arcs from one
-// atomic cursor, 11 ns each): t and 4-cliques at RMAT-20 329 -> 20.8 ms;
-// P7 at RMAT-18 280 -> 17.9 ms; P1 on 300007 vertices of degree 16
-// (2.4 million arcs) 27.4 -> 0.87 ms.
+// atomic cursor, 11 ns each): t and 4-cliques at RMAT-20 329 -> 7.3 ms;
+// P7 at RMAT-18 280 -> 8.3 ms; P1 on 300007 vertices of degree 16
+// (2.4 million arcs) 27.4 -> 0.79 ms.  Before the vertices with many lower
+// neighbours went to the large workgroups and the ranges were loaded 16 at a
+// time, 20.3 and 17.9 ms.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -51,19 +53,24 @@ constexpr int kWindowWords = kWindow / 32;
 constexpr int kLanesPerList = 16;        // lanes that walk one list
 constexpr int kUnroll = 4;               // loads in flight per lane
 
-// Classes by |N+(x)|: rows in LDS up to kRowsLdsMax, in the workgroup's
-// global slab above.  `words`: 64-bit words of row storage (U, then as many
-// columns of L as fit); `grab`: vertices per queue access.
+// Classes by the neighbours above and below x: rows in LDS up to 704 above,
+// in the workgroup's global slab beyond.  The lower neighbours cost a chain
+// of loads each and the highest ids have few neighbours but thousands below
+// them, so those go to the large workgroups: with classes by |N+(x)| alone
+// the 64 highest ids of RMAT-20 (1e6 lower neighbours, 0.3% of the items)
+// kept eight workgroups of 256 busy for 13 of the class's 15.4 ms.
+// `words`: 64-bit words of row storage (U, then as many columns of L as
+// fit); `grab`: most vertices per queue access.
 struct RowClass {
-  int max_out, threads, words, words_u, grab;
+  int max_out, max_below, threads, words, words_u, grab;
 };
+constexpr int kAnyBelow = 0x7fffffff;
 constexpr RowClass kRowClasses[kRowClassCount] = {
-    {64, 256, 1024, 64, 8},
-    {256, 512, 4096, 1024, 1},
-    {704, 1024, 13312, 7744, 1},
-    {0x7fffffff, 1024, 0, 0, 1},
+    {64, 256, 256, 320, 64, 8},
+    {256, 1024, 512, 4096, 1024, 1},
+    {704, kAnyBelow, 1024, 13312, 7744, 1},
+    {0x7fffffff, kAnyBelow, 1024, 0, 0, 1},
 };
-constexpr int kRowsLdsMax = 704;
 constexpr int kSlabL = 8;  // words of L per row in the global slab
 
 struct Locator {
@@ -112,6 +119,31 @@ __device__ __forceinline__ void stream_list(const int32_t *__restrict__ dcol,
     for (int u = 0; u < kUnroll; ++u) {
       const uint32_t qq = q + kLanesPerList * u;
       on_item(qq, loc.find(z[u], qq < e));
+    }
+  }
+}
+
+// Lists [0, cnt) dealt in turn to `groups` groups of 16 lanes (this one
+// `grp`), each up to 16 of its lists at a time: their ranges are loaded one per lane, so the
+// chain of loads to a range is paid once for all of them.  In turn, as the
+// lists are sorted by degree: with 16 in a row per group the two classes of
+// large workgroups took 8.9 ms on RMAT-20, in turn 4.9.
+// on_item(list, q, pos) as in stream_list.
+template <class R, class F>
+__device__ __forceinline__ void walk_lists(const int32_t *__restrict__ dcol,
+                                           int cnt, int grp, int groups,
+                                           int gl, const Locator &loc,
+                                           const R &range, const F &on_item) {
+  for (int k = grp; k < cnt; k += groups * kLanesPerList) {
+    const int mine = k + gl * groups;
+    uint32_t mb = 0, me = 0;
+    if (mine < cnt) range(mine, mb, me);
+    for (int i = 0, at = k; i < kLanesPerList && at < cnt;
+         ++i, at += groups) {
+      const uint32_t b = __shfl(mb, i, kLanesPerList);
+      const uint32_t e = __shfl(me, i, kLanesPerList);
+      stream_list(dcol, b, e, gl, loc,
+                  [&](uint32_t q, int pos) { on_item(at, q, pos); });
     }
   }
 }
@@ -173,15 +205,17 @@ __global__ __launch_bounds__(T) void census_rows(CensusArgs c, RowArgs r) {
   uint32_t *kacc = reinterpret_cast<uint32_t *>(slab + size_t(r.tri_cap) * 8);
   u64 k4 = 0, k5 = 0, kk = 0, tek = 0, tdk = 0, dp2 = 0, gem = 0, bad = 0;
   for (int i = tid; i < kWindowWords; i += T) s_bits[i] = 0;
-  for (;;) {
+  // The first vertices by workgroup, the rest from the queue.
+  const unsigned grab = static_cast<unsigned>(r.grab);
+  unsigned first = blockIdx.x * grab;
+  for (;; first = s_next) {
     __syncthreads();
-    if (tid == 0) s_next = atomicAdd(r.cursor, static_cast<unsigned>(r.grab));
-    __syncthreads();
-    const unsigned first = s_next;
-    if (first >= static_cast<unsigned>(r.count)) break;
-    const unsigned last =
-        min(first + static_cast<unsigned>(r.grab),
-            static_cast<unsigned>(r.count));
+    if (first >= r.count) break;
+    if (tid == 0) s_next = (gridDim.x * grab < r.count
+                                ? atomicAdd(r.cursor, grab)
+                                : r.count) +
+                           gridDim.x * grab;
+    const unsigned last = min(first + grab, r.count);
     for (unsigned ai = first; ai < last; ++ai) {
       const int32_t x = r.list[ai];
       const int64_t bx = c.drp[x];
@@ -216,44 +250,47 @@ __global__ __launch_bounds__(T) void census_rows(CensusArgs c, RowArgs r) {
       const Locator loc{s_bits, s_base, nb, c.winlo, s_low};
       u64 *U = rows;
       if (P >= 2) {
-        for (int i = grp; i < P; i += kGroups) {
+        auto above = [&](int i, uint32_t &b, uint32_t &e) {
           const int32_t y = nb[i];
-          const uint32_t b = static_cast<uint32_t>(c.drp[y]);
-          const uint32_t e = static_cast<uint32_t>(c.drp[y + 1]);
-          stream_list(c.dcol, b, e, gl, loc, [&](uint32_t q, int pos) {
-            if constexpr (CLIQUES) {
-              const bool hit = pos >= 0;
-              const u64 m = __ballot(hit);
-              if (m) {
-                const int lead = __builtin_ctzll(m);
-                unsigned o = 0;
-                if (lane == lead)
-                  o = atomicAdd(&s_nt, static_cast<unsigned>(__popcll(m)));
-                o = __shfl(o, lead, 64) + bits_below(m);
-                if (hit) {
-                  or_bit(U + size_t(i) * wu, pos);
-                  or_bit(U + size_t(pos) * wu, i);
-                  tri[o] = make_uint2(static_cast<unsigned>(i) |
-                                          static_cast<unsigned>(pos) << 16,
-                                      q);
+          b = static_cast<uint32_t>(c.drp[y]);
+          e = static_cast<uint32_t>(c.drp[y + 1]);
+        };
+        walk_lists(
+            c.dcol, P, grp, kGroups, gl, loc, above,
+            [&](int i, uint32_t q, int pos) {
+              if constexpr (CLIQUES) {
+                const bool hit = pos >= 0;
+                const u64 m = __ballot(hit);
+                if (m) {
+                  const int lead = __builtin_ctzll(m);
+                  unsigned o = 0;
+                  if (lane == lead)
+                    o = atomicAdd(&s_nt, static_cast<unsigned>(__popcll(m)));
+                  o = __shfl(o, lead, 64) + bits_below(m);
+                  if (hit) {
+                    or_bit(U + size_t(i) * wu, pos);
+                    or_bit(U + size_t(pos) * wu, i);
+                    tri[o] = make_uint2(static_cast<unsigned>(i) |
+                                            static_cast<unsigned>(pos) << 16,
+                                        q);
+                  }
                 }
+              } else if (pos >= 0) {
+                or_bit(U + size_t(i) * wu, pos);
+                atomicAdd(&cnt[pos], 1u);
               }
-            } else if (pos >= 0) {
-              or_bit(U + size_t(i) * wu, pos);
-              atomicAdd(&cnt[pos], 1u);
-            }
-          });
-        }
+            });
       }
+      // The tails past x of the lower neighbours' lists.
+      auto below = [&](int64_t k, uint32_t &b, uint32_t &e) {
+        b = c.arc[rb + k] + 1u;
+        e = static_cast<uint32_t>(c.drp[c.col[rb + k] + 1]);
+      };
       if constexpr (!CLIQUES) {
-        for (int k = grp; k < DL; k += kGroups) {
-          const int32_t w = c.col[rb + k];
-          const uint32_t b = c.arc[rb + k] + 1u;
-          const uint32_t e = static_cast<uint32_t>(c.drp[w + 1]);
-          stream_list(c.dcol, b, e, gl, loc, [&](uint32_t, int pos) {
-            if (pos >= 0) atomicAdd(&cnt[pos], 1u);
-          });
-        }
+        walk_lists(c.dcol, DL, grp, kGroups, gl, loc, below,
+                   [&](int, uint32_t, int pos) {
+                     if (pos >= 0) atomicAdd(&cnt[pos], 1u);
+                   });
         __syncthreads();
         for (int i = tid; i < P; i += T) {
           uint32_t t = LDS ? cnt[i]
@@ -289,14 +326,13 @@ __global__ __launch_bounds__(T) void census_rows(CensusArgs c, RowArgs r) {
           const int wc = (k1 - k0 + 63) >> 6;  // 0 when DL = 0
           for (int i = tid; i < P * wc; i += T) Lr[i] = 0;
           __syncthreads();
-          for (int k = k0 + grp; k < k1; k += kGroups) {
-            const int32_t w = c.col[rb + k];
-            const uint32_t b = c.arc[rb + k] + 1u;
-            const uint32_t e = static_cast<uint32_t>(c.drp[w + 1]);
-            stream_list(c.dcol, b, e, gl, loc, [&](uint32_t, int pos) {
-              if (pos >= 0) or_bit(Lr + size_t(pos) * wc, k - k0);
-            });
-          }
+          walk_lists(c.dcol, k1 - k0, grp, kGroups, gl, loc,
+                     [&](int k, uint32_t &b, uint32_t &e) {
+                       below(k0 + k, b, e);
+                     },
+                     [&](int k, uint32_t, int pos) {
+                       if (pos >= 0) or_bit(Lr + size_t(pos) * wc, k);
+                     });
           __syncthreads();
           for (int i = tid; i < P; i += T) {
             uint32_t t = 0;
@@ -422,10 +458,15 @@ __global__ __launch_bounds__(T) void census_rows(CensusArgs c, RowArgs r) {
 // Vertices per class, then their ids class by class, hubs first (the
 // vertex's index from the top of the id range): one atomic per class per
 // wave.
-__device__ __forceinline__ int row_class(int P) {
+__device__ __forceinline__ int row_class(const int64_t *__restrict__ drp,
+                                         const int32_t *__restrict__ deg,
+                                         int64_t v, int32_t n) {
+  if (v < 0 || v >= n) return -1;
+  const int P = static_cast<int>(drp[v + 1] - drp[v]);
   if (P < 1) return -1;
+  const int below = deg[v] - P;
   int k = 0;
-  while (P > kRowClasses[k].max_out) ++k;
+  while (P > kRowClasses[k].max_out || below > kRowClasses[k].max_below) ++k;
   return k;
 }
 
@@ -452,12 +493,11 @@ __device__ __forceinline__ ClassAt class_at(int k, int q, unsigned *s_wave) {
 }
 
 __global__ __launch_bounds__(kClassT) void rows_count(
-    const int64_t *__restrict__ drp, int32_t n,
-    unsigned *__restrict__ count) {
+    const int64_t *__restrict__ drp, const int32_t *__restrict__ deg,
+    int32_t n, unsigned *__restrict__ count) {
   __shared__ unsigned s_wave[kClassT / 64];
   const int64_t v = int64_t(blockIdx.x) * kClassT + threadIdx.x;
-  const int k =
-      v < n ? row_class(static_cast<int>(drp[v + 1] - drp[v])) : -1;
+  const int k = row_class(drp, deg, v, n);
   for (int q = 0; q < kRowClassCount; ++q) {
     const ClassAt c = class_at(k, q, s_wave);
     if (threadIdx.x == 0 && c.total) atomicAdd(&count[q], c.total);
@@ -465,15 +505,14 @@ __global__ __launch_bounds__(kClassT) void rows_count(
 }
 
 __global__ __launch_bounds__(kClassT) void rows_scatter(
-    const int64_t *__restrict__ drp, int32_t n,
-    const unsigned *__restrict__ count, unsigned *__restrict__ fill,
+    const int64_t *__restrict__ drp, const int32_t *__restrict__ deg,
+    int32_t n, const unsigned *__restrict__ count, unsigned *__restrict__ fill,
     int32_t *__restrict__ list) {
   __shared__ unsigned s_wave[kClassT / 64];
   __shared__ unsigned s_base;
   const int64_t v =
       int64_t(n) - 1 - (int64_t(blockIdx.x) * kClassT + threadIdx.x);
-  const int k =
-      v >= 0 ? row_class(static_cast<int>(drp[v + 1] - drp[v])) : -1;
+  const int k = row_class(drp, deg, v, n);
   unsigned start = 0;
   for (int q = 0; q < kRowClassCount; ++q) {
     const ClassAt c = class_at(k, q, s_wave);
@@ -520,11 +559,21 @@ size_t rows_slab_bytes(int cls, int64_t max_out) {
   return (b + 255) & ~size_t(255);
 }
 
+// Vertices per queue access: one while that leaves no workgroup more than
+// eight turns (RMAT-10 at eight each: 112 workgroups on 256 CUs).
+int rows_grab(int cls, int64_t count, bool cliques, int cus) {
+  const int64_t wgs = int64_t(cus) * rows_per_cu(cls, cliques);
+  return static_cast<int>(
+      std::max<int64_t>(1, std::min<int64_t>(kRowClasses[cls].grab,
+                                             count / (8 * wgs))));
+}
+
 int rows_grid(int cls, int64_t max_out, int64_t count, bool cliques,
               size_t budget, int cus) {
   if (count <= 0) return 0;
   const RowClass &k = kRowClasses[cls];
-  int64_t g = std::min<int64_t>((count + k.grab - 1) / k.grab,
+  const int64_t grab = rows_grab(cls, count, cliques, cus);
+  int64_t g = std::min<int64_t>((count + grab - 1) / grab,
                                 int64_t(cus) * rows_per_cu(cls, cliques));
   if (cliques || k.words == 0) {
     const size_t per = std::max<size_t>(rows_slab_bytes(cls, max_out), 1);
@@ -565,7 +614,7 @@ int census_rows_launch(const CensusArgs &c, const int64_t *cls_count,
     r.list = list + start[cls];
     r.count = static_cast<uint32_t>(cls_count[cls]);
     r.cursor = c.cursor + (cliques ? 8 : 4) + cls;
-    r.grab = k.grab;
+    r.grab = rows_grab(cls, cls_count[cls], cliques, cus);
     r.slab = slab;
     r.slab_bytes = rows_slab_bytes(cls, max_out);
     const int64_t P = std::min<int64_t>(max_out, k.max_out);
@@ -593,11 +642,13 @@ int census_rows_launch(const CensusArgs &c, const int64_t *cls_count,
   return 0;
 }
 
-int census_rows_classify(const int64_t *drp, int32_t n, unsigned *count,
-                         unsigned *fill, int32_t *list, hipStream_t s) {
+int census_rows_classify(const int64_t *drp, const int32_t *deg, int32_t n,
+                         unsigned *count, unsigned *fill, int32_t *list,
+                         hipStream_t s) {
   const int g = n / kClassT + 1;
-  hipLaunchKernelGGL(rows_count, dim3(g), dim3(kClassT), 0, s, drp, n, count);
-  hipLaunchKernelGGL(rows_scatter, dim3(g), dim3(kClassT), 0, s, drp, n,
+  hipLaunchKernelGGL(rows_count, dim3(g), dim3(kClassT), 0, s, drp, deg, n,
+                     count);
+  hipLaunchKernelGGL(rows_scatter, dim3(g), dim3(kClassT), 0, s, drp, deg, n,
                      count, fill, list);
   return hipGetLastError() == hipSuccess ? 0 : -1;
 }

@@ -63,3 +63,17 @@ def test_below_the_window(gpu_available):
     assert (both.pattern_count(1)[0] ==
             alone.pattern_count(1)[0] + 2 * half * comb(d, 3))
     assert both.tc_count()[0] == alone.tc_count()[0]
+
+
+@pytest.mark.parametrize("m", [255, 256, 257, 1023, 1024, 1025])
+def test_classes_by_lower_neighbours(gpu_available, m):
+    """K_5 joined to m independent vertices: four out-neighbours or fewer at
+    the edges of the classes by lower neighbours (256, 1024)."""
+    s = 5
+    rows = [np.delete(np.arange(s + m), v) for v in range(s)]
+    rows += [np.arange(s)] * m
+    dg = ma.DeviceGraph(_from_rows(rows), 0)
+    want = {1: s * comb(m, 3), 4: 0, 7: 2 * comb(s, 2) * comb(m, 3), 8: 0}
+    got = {p: dg.pattern_count(p)[0] for p in want}
+    dg.close()
+    assert got == want
