@@ -193,11 +193,11 @@ struct CensusGraph {
   DevView rowptr, col, deg, src, drp, dcol, arc, order;
   int64_t row_count[4] = {0, 0, 0, 0};
   // 4-cycle pass, built when a pattern first needs it: the first entry of
-  // every row in the counters' window, and the owners by kind and class
-  // (light, heavy), one list after the other.
+  // every row in the counters' window, and the owners by kind and class,
+  // one list after the other.
   bool c4_ready = false;
   DevBuf c4_win, c4_list;
-  uint32_t c4_count[3][2] = {{0, 0}, {0, 0}, {0, 0}};
+  uint32_t c4_count[3][4] = {};
   // Pair passes, likewise: pair-table slots and the n + 1 offsets of the
   // anchors' parts, the anchors by list (sizes in c5_count), and every row's
   // offsets of the fine windows.

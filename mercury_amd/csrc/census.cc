@@ -124,9 +124,9 @@ Need need_for(const mgpm_dgraph *dg, int passes, size_t budget) {
   // Heavy 4-cycle owners below the window (before the plan is built: as if
   // there were some).
   if (needs_c4(passes) && G.n > kRowWindow &&
-      (!cg.c4_ready || cg.c4_count[2][1])) {
+      (!cg.c4_ready || cg.c4_count[2][kC4Bits16])) {
     const size_t low = static_cast<size_t>(G.n - kRowWindow);
-    const size_t owners = cg.c4_ready ? cg.c4_count[2][1] : low;
+    const size_t owners = cg.c4_ready ? cg.c4_count[2][kC4Bits16] : low;
     k.c4_groups = static_cast<int>(std::max<size_t>(
         1, std::min<size_t>({size_t(dg->cus) * 2, owners,
                              kCensusC4Budget / (4 * low)})));
@@ -345,11 +345,11 @@ C4Plan c4_plan_of(const CensusGraph &cg) {
   C4Plan p;
   int32_t *at = cg.c4_list.as<int32_t>();
   for (int k = 0; k < kC4Kinds; ++k) {
-    p.light[k] = cg.c4_count[k][0];
-    p.heavy[k] = cg.c4_count[k][1];
-    p.light_list[k] = at;
-    p.heavy_list[k] = at + p.light[k];
-    at += size_t(p.light[k]) + p.heavy[k];
+    p.list[k] = at;
+    for (int q = 0; q < kC4Classes; ++q) {
+      p.count[k][q] = cg.c4_count[k][q];
+      at += p.count[k][q];
+    }
   }
   return p;
 }
@@ -366,7 +366,7 @@ int c4_layout(mgpm_dgraph *dg, hipStream_t s) {
   c.winlo = std::max<int32_t>(0, c.n - kRowWindow);
   const size_t n = std::max<size_t>(c.n, 1);
   DevBuf win, cls, fill;
-  unsigned sizes[2 * kC4Kinds];
+  unsigned sizes[kC4Kinds * kC4Classes];
   MGPM_HIP(win.alloc(n * sizeof(uint32_t)));
   MGPM_HIP(cls.alloc(n + static_cast<size_t>(c.winlo)));
   MGPM_HIP(fill.alloc(sizeof(sizes)));
@@ -383,7 +383,8 @@ int c4_layout(mgpm_dgraph *dg, hipStream_t s) {
   for (const unsigned x : sizes) total += x;
   MGPM_HIP(cg.c4_list.alloc(std::max<size_t>(total, 1) * sizeof(int32_t)));
   for (int k = 0; k < kC4Kinds; ++k)
-    for (int q = 0; q < 2; ++q) cg.c4_count[k][q] = sizes[2 * k + q];
+    for (int q = 0; q < kC4Classes; ++q)
+      cg.c4_count[k][q] = sizes[kC4Classes * k + q];
   if ((rc = zero(fill.p, sizeof(sizes), s))) return rc;
   if (census_c4_lists(c, cls.as<int8_t>(), fill.as<unsigned>(),
                       c4_plan_of(cg), s))

@@ -97,7 +97,7 @@ struct CensusArgs {
   const int32_t *order = nullptr;
   int32_t winlo = 0;
   // 4-cycle pass (census_c4.hip): first entry of every row in the window,
-  // queue counters (6, zeroed) and, for heavy owners below the window, per
+  // queue counters (12, zeroed) and, for heavy owners below the window, per
   // workgroup a dense counter array (winlo entries, zeroed; left zeroed).
   const uint32_t *win = nullptr;
   unsigned *c4_cursor = nullptr;
@@ -251,24 +251,26 @@ int census_rows_launch(const CensusArgs &c, const int64_t *cls_count,
 int census_sums_launch(const CensusArgs &c, int cus, hipStream_t s);
 
 // The 4-cycle pass's owners by kind (both ends in the window, the lower
-// one below it, both below) and class; the lists hold light and heavy ids.
+// one below it, both below) and class (light, or by the bits of a counter);
+// a kind's list holds its classes one after the other.
 constexpr int kC4Kinds = 3;
+enum C4Class : int { kC4Light, kC4Bits4, kC4Bits8, kC4Bits16, kC4Classes };
 struct C4Plan {
-  uint32_t light[kC4Kinds] = {0, 0, 0}, heavy[kC4Kinds] = {0, 0, 0};
-  int32_t *light_list[kC4Kinds] = {nullptr, nullptr, nullptr};
-  int32_t *heavy_list[kC4Kinds] = {nullptr, nullptr, nullptr};
+  uint32_t count[kC4Kinds][kC4Classes] = {};
+  int32_t *list[kC4Kinds] = {nullptr, nullptr, nullptr};
 };
 struct C4List {
   const int32_t *list = nullptr;
   uint32_t count = 0;
   unsigned *cursor = nullptr;
+  uint32_t grab = 1;  // owners per queue access
 };
 
 // Raises the dynamic-LDS limit of the 4-cycle kernels (once per process).
 int census_c4_init();
 // Enqueues the window offsets of the rows (n entries), the classes of the
-// owners (cls: n + winlo entries; class sizes {light, heavy} per kind into
-// fill, zeroed), and, with fill zeroed again, the lists of a plan that
+// owners (cls: n + winlo entries; the class sizes of each kind into fill,
+// zeroed), and, with fill zeroed again, the lists of a plan that
 // points at room for those sizes.
 int census_c4_window(const CensusArgs &c, uint32_t *win, hipStream_t s);
 int census_c4_classes(const CensusArgs &c, int8_t *cls, unsigned *fill,

@@ -44,3 +44,33 @@ def test_window_edges(gpu_available, n, draws):
         assert (dg.pattern_count(p)[0] == dg.pattern_count(
             p, ma.make_tune(pattern_census=-1))[0]), p
     dg.close()
+
+
+@pytest.mark.parametrize("c,d", [(2, 40), (15, 40), (16, 40), (255, 260),
+                                 (256, 260)])
+def test_counter_widths(gpu_available, c, d):
+    """Owners below the window with c middles (4, 8 and 16-bit counters take
+    up to 15, 255 and more) on a bipartite graph whose left vertex x sees
+    the right vertices x + 7j, j < d: owner i sees the left vertices i + 7j,
+    j < c, so i and the right vertex i + 7m have as many common neighbours as
+    m has sums j + k with j < c and k < d."""
+    half, owners = 33000, 4
+    x, j = np.arange(half)[:, None], 7 * np.arange(d)[None, :]
+    left = [np.sort(r) for r in owners + half + (x + j) % half]
+    right = [np.sort(r) for r in owners + (x - j) % half]
+    for i in range(owners):
+        for k in range(c):
+            left[i + 7 * k] = np.concatenate([[i], left[i + 7 * k]])
+    rows = [owners + i + 7 * np.arange(c) for i in range(owners)]
+    rows += left + right
+    rp = np.concatenate([[0], np.cumsum([len(r) for r in rows])])
+    dg = ma.DeviceGraph(
+        ma.Graph.from_csr(rp, np.concatenate(rows).astype(np.int32)), 0)
+    got = dg.pattern_count(4)[0]
+    dg.close()
+    sums = np.bincount((np.arange(c)[:, None] + np.arange(d)).ravel())
+    cycles = (half * sum(comb(d - k, 2) for k in range(1, d)) +
+              owners * sum(comb(int(s), 2) for s in sums))
+    paths = ((half * d - owners * c * d) * (d - 1) ** 2 +
+             owners * c * d * d * (d - 1) + owners * c * (c - 1) * d)
+    assert got == paths - 4 * cycles
