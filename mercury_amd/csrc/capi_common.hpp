@@ -191,7 +191,7 @@ struct CensusGraph {
   // out-neighbours grouped by the row passes' classes (sizes in row_count).
   DevBuf mem;
   DevView rowptr, col, deg, src, drp, dcol, arc, order;
-  int64_t row_count[4] = {0, 0, 0, 0};
+  int64_t row_count[5] = {0, 0, 0, 0, 0};
   // 4-cycle pass, built when a pattern first needs it: the first entry of
   // every row in the counters' window, and the owners by kind and class,
   // one list after the other.

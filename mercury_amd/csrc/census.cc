@@ -101,14 +101,14 @@ struct Need {
 size_t row_slab(const mgpm_dgraph *dg, int passes, int64_t max_out,
                 const int64_t *count) {
   size_t b = 0;
-  for (int cls = 0; cls < kRowClassCount; ++cls) {
-    const int64_t n = count ? count[cls] : dg->host->n;
+  for (int cls = 0; cls < kRowClassCount; ++cls)
     for (const bool cliques : {false, true})
       if (cliques ? is_k5(passes) : cls == kRowClassCount - 1)
         b = std::max(b, rows_slab_bytes(cls, max_out) *
-                            rows_grid(cls, max_out, n, cliques,
-                                      kCensusRowBudget, dg->cus));
-  }
+                            rows_grid(cls, max_out,
+                                      count ? rows_members(cls, count, cliques)
+                                            : dg->host->n,
+                                      cliques, kCensusRowBudget, dg->cus));
   return b;
 }
 

@@ -110,10 +110,11 @@ struct CensusArgs {
   unsigned long long *tv = nullptr;
 };
 
-// One class of vertices of the row passes (census_rows.hip): up to 64,
-// 256 and 704 out-neighbours with their bit rows in LDS, and the rest with
-// rows in the workgroup's slab.
-constexpr int kRowClassCount = 4;
+// Classes of vertices of the row passes (census_rows.hip): up to 64
+// out-neighbours, up to 32 neighbours on either side, up to 256 and 704
+// out-neighbours with their bit rows in LDS, and the rest with rows in the
+// workgroup's slab.
+constexpr int kRowClassCount = 5;
 constexpr int32_t kRowWindow = 65536;  // ids of the bitmap, the highest ones
 
 struct RowArgs {
@@ -228,6 +229,8 @@ int census_rows_init();
 // empty class) within `budget` bytes of slab, for graphs whose largest DAG
 // out-degree is max_out.  cliques: the pass of that setting.
 size_t rows_slab_bytes(int cls, int64_t max_out);
+// Vertices of class `cls` in a pass, of the class sizes count.
+int64_t rows_members(int cls, const int64_t *count, bool cliques);
 int rows_grid(int cls, int64_t max_out, int64_t count, bool cliques,
               size_t budget, int cus);
 

@@ -77,3 +77,23 @@ def test_classes_by_lower_neighbours(gpu_available, m):
     got = {p: dg.pattern_count(p)[0] for p in want}
     dg.close()
     assert got == want
+
+
+@pytest.mark.parametrize("copies", [40, 4200])
+@pytest.mark.parametrize("s,m", [(2, 1), (16, 8), (31, 2), (32, 1), (33, 1),
+                                 (34, 1), (20, 13), (8, 31), (8, 33)])
+def test_a_wave_per_vertex(gpu_available, s, m, copies):
+    """Copies of K_s joined to m vertices: at most 32 neighbours above and
+    below take a wave each where there are more than 4096 of them."""
+    n = s + m
+    rows = [np.delete(np.arange(n), v) for v in range(s)] + [np.arange(s)] * m
+    block = np.concatenate(rows)
+    rp = np.concatenate([[0], np.cumsum(np.tile([len(r) for r in rows],
+                                                copies))])
+    col = (block[None, :] + n * np.arange(copies)[:, None]).ravel()
+    dg = ma.DeviceGraph(ma.Graph.from_csr(rp, col.astype(np.int32)), 0)
+    want = {1: copies * s * comb(m, 3), 4: 0,
+            7: 2 * copies * comb(s, 2) * comb(m, 3), 8: 0}
+    got = {p: dg.pattern_count(p)[0] for p in want}
+    dg.close()
+    assert got == want
