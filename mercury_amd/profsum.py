@@ -22,6 +22,7 @@ from pathlib import Path
 
 COUNTING = ("tc_wave_tables", "tc_half_tables", "tc_block_tables",
             "tc_global_search", "pattern_", "batch_kernel")
+COUNTING_EXACT = ("hub_count", "hub_rest")  # hub_counts prepares
 
 
 def _short(name: str) -> str:
@@ -66,7 +67,7 @@ def _copy_kib(d: str, counter: str) -> float:
 def _counting_kib(d: str, counter: str) -> float:
     return sum(v.get(counter, 0.0)
                for (_, k), v in counter_per_dispatch(d).items()
-               if any(c in k for c in COUNTING))
+               if k in COUNTING_EXACT or any(c in k for c in COUNTING))
 
 
 def traffic(a) -> dict:
