@@ -40,6 +40,7 @@
 
 #include "census.hpp"
 #include "choose.hpp"
+#include "lanes.hpp"
 #include "wave.hpp"
 
 namespace mgpm {
@@ -112,19 +113,15 @@ __device__ __forceinline__ void walk(const CensusArgs &c, uint32_t i0,
     for (uint32_t x = 0, i = k; x < kLanes && i < cnt; ++x, i += groups) {
       const uint32_t b = __shfl(r.b, static_cast<int>(x), kLanes);
       const uint32_t e = __shfl(r.e, static_cast<int>(x), kLanes);
-      for (uint32_t j = b + gl; j < e; j += kLanes * kUnroll) {
-        int32_t w[kUnroll];
+      lane_walk<kLanes, kUnroll>(
+          b, e, static_cast<uint32_t>(gl),
+          [&](const uint32_t(&j)[kUnroll], const bool(&ok)[kUnroll]) {
+            int32_t w[kUnroll];
 #pragma unroll
-        for (int q = 0; q < kUnroll; ++q) {
-          const uint32_t jj = j + kLanes * q;
-          w[q] = c.col[jj < e ? jj : j];
-        }
+            for (int q = 0; q < kUnroll; ++q) w[q] = c.col[j[q]];
 #pragma unroll
-        for (int q = 0; q < kUnroll; ++q) {
-          const uint32_t jj = j + kLanes * q;
-          on_item(i0 + i, jj, w[q], jj < e);
-        }
-      }
+            for (int q = 0; q < kUnroll; ++q) on_item(i0 + i, j[q], w[q], ok[q]);
+          });
     }
   }
 }
