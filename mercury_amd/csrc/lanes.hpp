@@ -29,4 +29,17 @@ MGPM_HD void lane_walk(uint32_t b, uint32_t e, uint32_t lane, const F &step) {
   }
 }
 
+// Where a search of the sorted entries [lo, end) of an array starts and how
+// many entries it has left, one at least: searches in lockstep all read while
+// the longest one lasts.  One that has nothing to find (not ok, or an empty
+// list) stays on the array's first entry: a list that is empty because no arc
+// follows it begins past the last one.
+struct Window {
+  uint32_t lo, len;
+};
+MGPM_HD Window search_window(uint32_t lo, uint32_t end, bool ok) {
+  if (!ok || end <= lo) return {0u, 1u};
+  return {lo, end - lo};
+}
+
 }  // namespace mgpm

@@ -37,6 +37,7 @@
 
 #include <algorithm>
 
+#include "lanes.hpp"
 #include "tc_hub.hpp"
 #include "wave.hpp"
 
@@ -349,10 +350,11 @@ __global__ __launch_bounds__(kWaves * 64) void hub_rest(TcHubPlan p,
         ok[k] = q < s * s && j > i;
         const int32_t b = N[ok[k] ? i : 0];
         z[k] = N[ok[k] ? j : 0];
-        lo[k] = static_cast<uint32_t>(p.drp[b]);
-        len[k] = p.split[b] - lo[k];
-        ok[k] = ok[k] && len[k] > 0;
-        if (!ok[k]) len[k] = 1;  // one element at a valid address
+        const uint32_t lb = static_cast<uint32_t>(p.drp[b]);
+        ok[k] = ok[k] && p.split[b] > lb;
+        const Window w = search_window(lb, p.split[b], ok[k]);
+        lo[k] = w.lo;
+        len[k] = w.len;
         most = max(most, len[k]);
       }
       // The last element <= z of each list, every window halving until it
