@@ -169,7 +169,7 @@ int BatchExec::plan(const mgpm_query *q, int nq, uint64_t max_bytes) {
       return fail(MGPM_ERR_PATTERN, "Not support.");
   }
   // Checked before anything is allocated or built.
-  if (growth(q, nq) > max_bytes)
+  if (max_bytes != UINT64_MAX && growth(q, nq) > max_bytes)
     return fail(MGPM_ERR_CAPACITY, "batch workspace exceeds the HBM budget");
   queries_.assign(static_cast<size_t>(nq), Planned{});
   jobs_.clear();

@@ -4,8 +4,10 @@
 #include <hip/hip_runtime_api.h>
 
 #include <algorithm>
+#include <atomic>
 #include <chrono>
 #include <memory>
+#include <mutex>
 #include <string>
 #include <utility>
 #include <vector>
@@ -214,9 +216,9 @@ struct CensusGraph {
 // The triangle count's hub plan (tc_hub.cc), built on the first count that
 // takes it and kept with the graph.
 struct TcHub {
-  int wanted = -1;  // the rule's answer (-1: not asked yet)
+  std::atomic<int> wanted{-1};  // the rule's answer (-1: not asked yet)
   bool off = false;  // the autotuner measured a table plan as faster
-  bool ready = false;
+  std::atomic<bool> ready{false};
   TcHubPlan plan;
   DevBuf mem;   // everything plan points at, and own
   DevView own;  // result and queue of single counts (zero between them)
@@ -305,7 +307,8 @@ int census_combine(int pattern, const unsigned long long *acc,
 // Device bytes of a census workspace for these passes on this graph
 // (before the graph's census DAG exists: a bound that includes it).
 uint64_t census_work_bytes(const mgpm_dgraph *dg, int passes, size_t budget);
-// The census graph alone (relabelled CSR, DAG, arcs), built once.
+// The census graph alone (relabelled CSR, DAG, arcs), built once; the caller
+// holds prep_mu.
 int census_graph_ready(mgpm_dgraph *dg, hipStream_t s);
 // Whether triangle counts of the graph go against hub bitmaps unless the
 // caller sets a triangle knob; the plan for it, built once.
@@ -338,6 +341,9 @@ struct mgpm_dgraph {
   mgpm::DagResident dag;
   mgpm::CensusGraph census;            // DAG of the census
   mgpm::TcHub hub;                     // hub plan of the triangle count
+  // Held while the census graph, its layouts or the hub plan are built: what
+  // is ready is only read, by batches of several threads too.
+  std::mutex prep_mu;
   mgpm::DevBuf scratch;               // queues + result counters
   unsigned long long *pinned = nullptr;  // host mirror of results
   hipEvent_t ev0 = nullptr, ev1 = nullptr;

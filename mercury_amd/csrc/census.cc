@@ -491,6 +491,7 @@ int census_graph_ready(mgpm_dgraph *dg, hipStream_t s) {
 }
 
 int census_graph_prepare(mgpm_dgraph *dg, hipStream_t s) {
+  std::lock_guard<std::mutex> lk(dg->prep_mu);
   int rc = graph_ready(dg, s);
   if (rc) return rc;
   if ((rc = c4_layout(dg, s))) return rc;
@@ -509,10 +510,13 @@ int census_passes(int pattern) {
 
 int census_prepare(mgpm_dgraph *dg, int passes, CensusWork &w,
                    hipStream_t s) {
-  int rc = graph_ready(dg, s);
-  if (rc) return rc;
-  if (needs_c4(passes) && (rc = c4_layout(dg, s))) return rc;
-  if (is_full5(passes) && (rc = pairs_layout(dg, s))) return rc;
+  {
+    std::lock_guard<std::mutex> lk(dg->prep_mu);
+    int rc = graph_ready(dg, s);
+    if (rc) return rc;
+    if (needs_c4(passes) && (rc = c4_layout(dg, s))) return rc;
+    if (is_full5(passes) && (rc = pairs_layout(dg, s))) return rc;
+  }
   return work_grow(w, need_for(dg, passes, w.budget), s);
 }
 

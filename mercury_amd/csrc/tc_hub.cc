@@ -83,6 +83,7 @@ bool tc_hub_wanted(mgpm_dgraph *dg) {
 
 int tc_hub_prepare(mgpm_dgraph *dg, hipStream_t s) {
   TcHub &h = dg->hub;
+  std::lock_guard<std::mutex> lk(dg->prep_mu);
   if (h.ready) return MGPM_OK;
   int rc = census_graph_ready(dg, s);
   if (rc) return rc;
