@@ -183,11 +183,10 @@ int BatchExec::plan(const mgpm_query *q, int nq, uint64_t max_bytes) {
     if (p == MGPM_TC) {
       pq.cost = query_cost(g, p);
       // The hub plan is kept with the graph, like the census graph it is
-      // made from; without the memory the table plan counts.
-      if (census_ && !g->hub.off && tc_hub_wanted(g)) {
-        const int rc = tc_hub_prepare(g, nullptr);
-        if (rc == MGPM_ERR_NOMEM) (void)hipGetLastError();
-        else if (rc) return rc;
+      // made from.
+      if (census_) {
+        const int rc = tc_hub_use(g, nullptr, &pq.hub);
+        if (rc) return rc;
       }
     } else if (census_) {
       auto it = job_of.find(g);
@@ -303,7 +302,7 @@ int BatchExec::enqueue(hipStream_t s, bool copy_back) {
       }
       const int i = u;
       const Planned &qp = queries_[i];
-      if (qp.pattern == MGPM_TC && qp.g->hub.ready && !qp.g->hub.off) {
+      if (qp.hub) {
         HubOut out;
         out.result = counters + 2 * i;
         if (tc_hub_launch(qp.g->hub.plan, out, cus_, ls))

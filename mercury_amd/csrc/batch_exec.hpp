@@ -72,6 +72,7 @@ class BatchExec {
     int pattern = 0;
     uint64_t cost = 0;
     int job = -1;  // census job that gives its count (-1: own kernels)
+    bool hub = false;  // a triangle count against hub bitmaps
   };
   // One census run per graph in the batch, with the union of the passes its
   // queries need.

@@ -598,20 +598,12 @@ int mgpm_tc_count(mgpm_dgraph *dg, const mgpm_tune *tune, void *stream,
   hipStream_t s = static_cast<hipStream_t>(stream);
   double prep = 0;
   // Hub bitmaps where hubs dominate, unless a triangle knob asks for the
-  // table plan; the plan is built on the first such count.  One that cannot
-  // be allocated is skipped (the failed allocation's error is cleared so
-  // that the launch check does not see it).
-  bool hub = !tc_knob_set(tune) && !dg->hub.off && tc_hub_wanted(dg);
-  if (hub && !dg->hub.ready) {
-    const auto tp = std::chrono::steady_clock::now();
-    rc = tc_hub_prepare(dg, s);
-    if (rc == MGPM_ERR_NOMEM) {
-      (void)hipGetLastError();
-      hub = false;
-    } else if (rc) {
-      return rc;
-    }
-    prep = ms_since(tp);
+  // table plan; the plan is built on the first such count.
+  bool hub = false;
+  if (!tc_knob_set(tune)) {
+    const bool had = dg->hub.ready;
+    if ((rc = tc_hub_use(dg, s, &hub))) return rc;
+    if (hub && !had) prep = ms_since(t0);
   }
   if (hub) {
     MGPM_HIP(hipEventRecord(dg->ev0, s));

@@ -97,6 +97,7 @@ class DevArena {
         v.first->p = static_cast<char *>(mem.p) + v.second;
     return e;
   }
+  size_t bytes() const { return total_; }
 
  private:
   std::vector<std::pair<DevView *, size_t>> views_;
@@ -218,6 +219,8 @@ struct CensusGraph {
 struct TcHub {
   std::atomic<int> wanted{-1};  // the rule's answer (-1: not asked yet)
   bool off = false;  // the autotuner measured a table plan as faster
+  bool refused = false;  // its server has no memory for it
+  size_t short_of = 0;  // free device bytes when it could not be allocated
   std::atomic<bool> ready{false};
   TcHubPlan plan;
   DevBuf mem;   // everything plan points at, and own
@@ -310,10 +313,18 @@ uint64_t census_work_bytes(const mgpm_dgraph *dg, int passes, size_t budget);
 // The census graph alone (relabelled CSR, DAG, arcs), built once; the caller
 // holds prep_mu.
 int census_graph_ready(mgpm_dgraph *dg, hipStream_t s);
+// Drops a census graph that nothing was built on; the caller holds prep_mu.
+void census_graph_drop(mgpm_dgraph *dg);
 // Whether triangle counts of the graph go against hub bitmaps unless the
-// caller sets a triangle knob; the plan for it, built once.
+// caller sets a triangle knob, and the device bytes its plan keeps.
 bool tc_hub_wanted(mgpm_dgraph *dg);
-int tc_hub_prepare(mgpm_dgraph *dg, hipStream_t s);
+uint64_t tc_hub_bytes(const mgpm_dgraph *dg);
+// The plan, built once: *use says whether counts take it.  The table plan
+// counts what it does not, so a plan that is not wanted or that cannot be
+// allocated is no error; the latter is tried again when more memory is free.
+int tc_hub_use(mgpm_dgraph *dg, hipStream_t s, bool *use);
+// Frees the plan for good; no count that takes it may be in flight.
+void tc_hub_release(mgpm_dgraph *dg);
 // Rebuilds the resident triangle plan where it was built (host or device).
 int tc_replan(mgpm_dgraph *dg, const TcPlanParams &params, hipStream_t s);
 // Builds pattern `pattern`'s plan if missing or if `split` (0 = the

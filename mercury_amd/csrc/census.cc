@@ -490,6 +490,11 @@ int census_graph_ready(mgpm_dgraph *dg, hipStream_t s) {
   return graph_ready(dg, s);
 }
 
+void census_graph_drop(mgpm_dgraph *dg) {
+  dg->census.ready = false;
+  dg->census.mem.reset();
+}
+
 int census_graph_prepare(mgpm_dgraph *dg, hipStream_t s) {
   std::lock_guard<std::mutex> lk(dg->prep_mu);
   int rc = graph_ready(dg, s);

@@ -100,11 +100,43 @@ uint64_t room_for(const mgpm_server *s) {
   return s->budget > used ? s->budget - used : 0;
 }
 
+// Whether a batch in flight counts triangles of graph `gid` (lock held).
+bool hub_in_flight(const mgpm_server *s, int32_t gid) {
+  for (const Slot &sl : s->slots)
+    if (sl.busy)
+      for (uint64_t t : sl.tickets) {
+        const auto it = s->reqs.find(t);
+        if (it != s->reqs.end() && it->second.graph == gid &&
+            it->second.pattern == MGPM_TC)
+          return true;
+      }
+  return false;
+}
+
+// Hub plans take memory that nothing else needs: frees those that no batch
+// in flight uses until `bytes` fit the budget, and keeps new batches off the
+// others (lock held).  Returns whether the bytes fit.
+bool make_room(mgpm_server *s, uint64_t bytes) {
+  uint64_t hubs = 0;
+  for (const mgpm_dgraph *g : s->graphs) hubs += g->hub.bytes();
+  if (bytes > room_for(s) + hubs) return false;  // not without them either
+  for (size_t i = 0; i < s->graphs.size() && bytes > room_for(s); ++i) {
+    mgpm_dgraph *g = s->graphs[i];
+    const uint64_t b = g->hub.bytes();
+    if (!b) continue;
+    g->hub.refused = true;
+    if (hub_in_flight(s, static_cast<int32_t>(i))) continue;
+    tc_hub_release(g);
+    s->resident -= b;
+  }
+  return bytes <= room_for(s);
+}
+
 // Takes pending requests in arrival order for free slot `sl` while their
 // workspaces fit the budget (server lock held).  The first request that
 // does not fit stops the intake and waits: when no batch is in flight, the
-// idle slots' workspaces are released for it, and if it still cannot fit
-// it fails alone (MGPM_ERR_CAPACITY) while the rest keep their turn.
+// idle slots' workspaces and the graphs' hub plans are released for it, and
+// if it still cannot fit it fails alone (MGPM_ERR_CAPACITY) while the rest keep their turn.
 std::vector<uint64_t> admit(mgpm_server *s, Slot &sl) {
   std::vector<uint64_t> take;
   uint64_t wc = 0, ws = 0;
@@ -135,7 +167,7 @@ std::vector<uint64_t> admit(mgpm_server *s, Slot &sl) {
       freed += b - o.exec.footprint();
     }
     s->workspace -= std::min(s->workspace, freed);
-    if (sl.exec.growth_for(c2, s2, nq) <= room_for(s)) continue;
+    if (make_room(s, sl.exec.growth_for(c2, s2, nq))) continue;
     s->pending.pop_front();  // can never fit: fails alone
     s->st.deferred_failed++;
     finish(s, t, 0, MGPM_ERR_CAPACITY, 0, Clock::now());
@@ -260,18 +292,12 @@ int mgpm_server_add_graph(mgpm_server *s, const mgpm_graph *g,
     // Upload (TC plan) and build what the pattern counts keep with the
     // graph -- the census DAG and pair-table layout, or every pattern's
     // per-edge plan -- then admit by footprint (the slots hold the
-    // workspaces, so the graph holds none).
+    // workspaces, so the graph holds none).  The hub plan comes after, where
+    // the budget has room for it: the table plan gives the same count.
     mgpm_dgraph *dg = nullptr;
     if ((rc = mgpm_dgraph_upload(g, s->cfg.device, nullptr, &dg))) return rc;
     if (s->cfg.pattern_census >= 0) {
       rc = census_graph_prepare(dg, nullptr);
-      if (!rc && tc_hub_wanted(dg)) {
-        rc = tc_hub_prepare(dg, nullptr);
-        if (rc == MGPM_ERR_NOMEM) {  // the table plan counts triangles
-          (void)hipGetLastError();
-          rc = MGPM_OK;
-        }
-      }
     } else {
       for (int p = MGPM_P1; p <= MGPM_P8 && !rc; ++p)
         rc = pattern_make_resident(dg, nullptr, p);
@@ -282,12 +308,40 @@ int mgpm_server_add_graph(mgpm_server *s, const mgpm_graph *g,
     }
     uint64_t bytes = 0;
     mgpm_dgraph_footprint(dg, &bytes);
-    std::lock_guard<std::mutex> lk(s->mu);
-    if (s->resident + s->workspace + bytes > s->budget) {
-      mgpm_dgraph_free(dg);
-      return fail(MGPM_ERR_CAPACITY, "graph does not fit the HBM budget");
+    std::unique_lock<std::mutex> lk(s->mu);
+    while (bytes > room_for(s) && !make_room(s, bytes)) {
+      // Hub plans in use go when their batches are done.
+      uint64_t hubs = 0;
+      for (const mgpm_dgraph *o : s->graphs) hubs += o->hub.bytes();
+      if (bytes > room_for(s) + hubs) {
+        mgpm_dgraph_free(dg);
+        return fail(MGPM_ERR_CAPACITY, "graph does not fit the HBM budget");
+      }
+      s->cv_done.wait(lk);
     }
     s->resident += bytes;
+    uint64_t hub = 0;  // reserved while it is built
+    if (s->cfg.pattern_census >= 0 && tc_hub_wanted(dg)) {
+      hub = tc_hub_bytes(dg);
+      if (hub > room_for(s)) hub = 0;
+    }
+    if (hub) {
+      s->resident += hub;
+      lk.unlock();
+      bool use = false;
+      rc = tc_hub_use(dg, nullptr, &use);
+      if (!use) tc_hub_release(dg);
+      lk.lock();
+      s->resident -= hub - dg->hub.bytes();
+      if (rc) {
+        s->resident -= bytes;
+        lk.unlock();
+        mgpm_dgraph_free(dg);
+        return rc;
+      }
+    } else {
+      dg->hub.refused = true;  // counts do not build it either
+    }
     s->graphs.push_back(dg);
     s->graph_bytes.push_back(bytes);
     *graph_id = static_cast<int32_t>(s->graphs.size()) - 1;

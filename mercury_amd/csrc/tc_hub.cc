@@ -73,45 +73,52 @@ bool hubs_pay(const mgpm_dgraph *dg) {
   return hubs_hold(g, 1, long_lists ? 4 : 2);
 }
 
-}  // namespace
+// What a plan keeps: its sizes in p, its arrays added to `keep`.
+struct HubKeep {
+  DevView rows, owner, part, bound, start, rest, split, own;
+};
+constexpr size_t kOwnWords = kHubQueueStride + kHubQueueWords;
 
-bool tc_hub_wanted(mgpm_dgraph *dg) {
-  TcHub &h = dg->hub;
-  if (h.wanted < 0) h.wanted = hubs_pay(dg) ? 1 : 0;
-  return h.wanted > 0;
+uint32_t runs_of(const mgpm_dgraph *dg) {
+  return static_cast<uint32_t>((dg->host->nnz / 2 + kHubRun - 1) / kHubRun);
 }
 
-int tc_hub_prepare(mgpm_dgraph *dg, hipStream_t s) {
+void keep_layout(const mgpm_dgraph *dg, TcHubPlan &p, HubKeep &k,
+                 DevArena &keep) {
+  const int64_t m = dg->host->nnz / 2;
+  const size_t n1 = static_cast<size_t>(dg->host->n) + 1;
+  p.n = static_cast<uint32_t>(dg->host->n);
+  p.nparts = static_cast<uint32_t>(m);
+  p.blocks = block_count(p.nparts, runs_of(dg), dg->cus);
+  // Chunks of all rows: every row rounded up, and the padding chunk.
+  const size_t nchunks = static_cast<size_t>(m) / kHubChunk + n1;
+  keep.add(k.rows, nchunks * kHubChunk * 2);
+  keep.add(k.owner, n1 * sizeof(HubOwner));
+  keep.add(k.part, static_cast<size_t>(m) * sizeof(HubPartner));
+  keep.add(k.bound, (size_t(p.blocks) + 1) * 4);
+  keep.add(k.start, (size_t(p.blocks) + 1) * 4);
+  keep.add(k.rest, n1 * 4);
+  keep.add(k.split, n1 * 4);
+  keep.add(k.own, kOwnWords * 4);
+}
+
+// Builds the plan (prep_mu held).
+int prepare(mgpm_dgraph *dg, hipStream_t s) {
   TcHub &h = dg->hub;
-  std::lock_guard<std::mutex> lk(dg->prep_mu);
-  if (h.ready) return MGPM_OK;
   int rc = census_graph_ready(dg, s);
   if (rc) return rc;
   const CensusGraph &cg = dg->census;
   const int32_t n = dg->host->n;
-  const int64_t nnz = dg->host->nnz, m = nnz / 2;
+  const int64_t nnz = dg->host->nnz;
   const int32_t hublo = std::max<int32_t>(0, n - kHubIds);
   const size_t n1 = static_cast<size_t>(n) + 1;
-  const uint32_t runs = static_cast<uint32_t>((m + kHubRun - 1) / kHubRun);
+  const uint32_t runs = runs_of(dg);
   const int64_t *drp = cg.drp.as<int64_t>();
   const int32_t *dcol = cg.dcol.as<int32_t>();
   TcHubPlan p;
-  p.n = static_cast<uint32_t>(n);
-  p.nparts = static_cast<uint32_t>(m);
-  p.blocks = block_count(p.nparts, runs, dg->cus);
-  // Chunks of all rows: every row rounded up, and the padding chunk.
-  const size_t nchunks = static_cast<size_t>(m) / kHubChunk + n1;
-  constexpr size_t kOwnWords = kHubQueueStride + kHubQueueWords;
-  DevView rows, owner, part, bound, start, rest, split;
+  HubKeep k;
   DevArena keep;
-  keep.add(rows, nchunks * kHubChunk * 2);
-  keep.add(owner, n1 * sizeof(HubOwner));
-  keep.add(part, static_cast<size_t>(m) * sizeof(HubPartner));
-  keep.add(bound, (size_t(p.blocks) + 1) * 4);
-  keep.add(start, (size_t(p.blocks) + 1) * 4);
-  keep.add(rest, n1 * 4);
-  keep.add(split, n1 * 4);
-  keep.add(h.own, kOwnWords * 4);
+  keep_layout(dg, p, k, keep);
   DevBuf mem, tmp_mem;  // mem becomes h.mem when it is complete
   DevView rowbase, chunks, flag, pos, meta, cost, prefix, total, scan;
   const size_t sb = tc_hub_scan_bytes(n, runs);
@@ -125,31 +132,31 @@ int tc_hub_prepare(mgpm_dgraph *dg, hipStream_t s) {
   work.add(scan, sb);
   MGPM_HIP(keep.alloc(mem));
   MGPM_HIP(work.alloc(tmp_mem));
-  p.rows = rows.p;
-  p.owner = owner.as<HubOwner>();
-  p.part = part.as<HubPartner>();
-  p.bound = bound.as<uint32_t>();
-  p.start = start.as<uint32_t>();
-  p.rest = rest.as<int32_t>();
+  p.rows = k.rows.p;
+  p.owner = k.owner.as<HubOwner>();
+  p.part = k.part.as<HubPartner>();
+  p.bound = k.bound.as<uint32_t>();
+  p.start = k.start.as<uint32_t>();
+  p.rest = k.rest.as<int32_t>();
   p.drp = drp;
   p.dcol = dcol;
-  p.split = split.as<uint32_t>();
+  p.split = k.split.as<uint32_t>();
   const uint32_t *owners = pos.as<uint32_t>() + n;
-  if (tc_hub_counts(drp, dcol, n, hublo, split.as<uint32_t>(),
+  if (tc_hub_counts(drp, dcol, n, hublo, k.split.as<uint32_t>(),
                     chunks.as<uint32_t>(), s) ||
       tc_hub_scan(chunks.as<uint32_t>(), rowbase.as<uint32_t>(), n, scan.p,
                   sb, s) ||
-      device_zero(total.p, 1, s) || device_zero(h.own.p, kOwnWords, s) ||
+      device_zero(total.p, 1, s) || device_zero(k.own.p, kOwnWords, s) ||
       tc_hub_fill(cg.rowptr.as<int64_t>(), cg.col.as<int32_t>(),
                   cg.src.as<int32_t>(), nnz, drp, dcol, cg.arc.as<uint32_t>(),
-                  n, split.as<uint32_t>(), rowbase.as<uint32_t>(), rows.p,
+                  n, k.split.as<uint32_t>(), rowbase.as<uint32_t>(), k.rows.p,
                   flag.as<uint32_t>(), pos.as<uint32_t>(), meta.p,
-                  owner.as<HubOwner>(), part.as<HubPartner>(),
-                  rest.as<int32_t>(), total.as<uint32_t>(), scan.p, sb,
+                  k.owner.as<HubOwner>(), k.part.as<HubPartner>(),
+                  k.rest.as<int32_t>(), total.as<uint32_t>(), scan.p, sb,
                   dg->cus, s) ||
       tc_hub_blocks(p, owners, runs, cost.as<unsigned long long>(),
                     prefix.as<unsigned long long>(), scan.p, sb,
-                    bound.as<uint32_t>(), start.as<uint32_t>(), s))
+                    k.bound.as<uint32_t>(), k.start.as<uint32_t>(), s))
     return fail(MGPM_ERR_HIP, "hub plan kernel launch failed");
   MGPM_HIP(hipMemcpyAsync(&p.nrest, total.p, 4, hipMemcpyDeviceToHost, s));
   MGPM_HIP(hipMemcpyAsync(&p.owners, owners, 4, hipMemcpyDeviceToHost, s));
@@ -157,8 +164,61 @@ int tc_hub_prepare(mgpm_dgraph *dg, hipStream_t s) {
   if (p.owners == 0) p.blocks = 0;  // no arc follows another: no triangle
   h.mem.swap(mem);
   h.plan = p;
+  h.own = k.own;
   h.ready = true;
   return MGPM_OK;
+}
+
+}  // namespace
+
+bool tc_hub_wanted(mgpm_dgraph *dg) {
+  TcHub &h = dg->hub;
+  if (h.off || h.refused) return false;
+  if (h.wanted < 0) h.wanted = hubs_pay(dg) ? 1 : 0;
+  return h.wanted > 0;
+}
+
+uint64_t tc_hub_bytes(const mgpm_dgraph *dg) {
+  TcHubPlan p;
+  HubKeep k;
+  DevArena keep;
+  keep_layout(dg, p, k, keep);
+  return keep.bytes();
+}
+
+int tc_hub_use(mgpm_dgraph *dg, hipStream_t s, bool *use) {
+  TcHub &h = dg->hub;
+  *use = false;
+  if (!tc_hub_wanted(dg)) return MGPM_OK;
+  if ((*use = h.ready)) return MGPM_OK;
+  std::lock_guard<std::mutex> lk(dg->prep_mu);
+  if ((*use = h.ready)) return MGPM_OK;
+  size_t free_b = 0, total_b = 0;
+  if (h.short_of) {
+    MGPM_HIP(hipMemGetInfo(&free_b, &total_b));
+    if (free_b <= h.short_of) return MGPM_OK;
+  }
+  const bool had = dg->census.ready;
+  const int rc = prepare(dg, s);
+  if (rc == MGPM_ERR_NOMEM) {
+    // Cleared, so that no launch check sees it; without the census graph if
+    // that was built for this plan alone.
+    (void)hipGetLastError();
+    if (!had) census_graph_drop(dg);
+    MGPM_HIP(hipMemGetInfo(&free_b, &total_b));
+    h.short_of = std::max<size_t>(free_b, 1);
+    return MGPM_OK;
+  }
+  *use = rc == MGPM_OK;
+  return rc;
+}
+
+void tc_hub_release(mgpm_dgraph *dg) {
+  std::lock_guard<std::mutex> lk(dg->prep_mu);
+  TcHub &h = dg->hub;
+  h.refused = true;
+  h.ready = false;
+  h.mem.reset();
 }
 
 }  // namespace mgpm
