@@ -202,10 +202,11 @@ struct CensusGraph {
   DevBuf c4_win, c4_list;
   uint32_t c4_count[3][4] = {};
   // Pair passes, likewise: pair-table slots and the n + 1 offsets of the
-  // anchors' parts, the anchors by list (sizes in c5_count), and every row's
-  // offsets of the fine windows.
+  // anchors' parts, the anchors by list (sizes in c5_count), and the offsets
+  // of the fine windows in the rows from c5_first on (Census5Args::woff).
   bool pairs_ready = false;
   uint64_t tab_total = 0;
+  int32_t c5_first = 0;
   DevBuf tab_off, c5_list, c5_woff;
   uint32_t c5_count[6] = {0, 0, 0, 0, 0, 0};
   size_t bytes() const {

@@ -271,6 +271,7 @@ Census5Args args5_of(mgpm_dgraph *dg, CensusWork &w, const Need &k) {
   c.winlo = std::max<int32_t>(0, c.n - kRowWindow);
   c.nf = census5_fine_windows(c.n, c.winlo);
   c.win = cg.c4_win.as<uint32_t>();
+  c.first = cg.c5_first;
   c.woff = cg.c5_woff.as<uint16_t>();
   c.lo = w.lo.as<uint32_t>();
   c.mask = w.mask.as<unsigned long long>();
@@ -422,13 +423,14 @@ int pairs_layout(mgpm_dgraph *dg, hipStream_t s) {
   c.groups = static_cast<int>(std::max<size_t>(
       1, std::min<size_t>(size_t(dg->cus) * 2,
                           (kCensus5Budget / 4) / (4 * below))));
-  constexpr size_t kCls = 3 * kC5Lists * sizeof(unsigned);
+  constexpr size_t kCls = (3 * kC5Lists + 1) * sizeof(unsigned);
   size_t sb = 0;
   if (census5_scan_bytes(int64_t(n1), &sb))
     return fail(MGPM_ERR_HIP, "scan size query");
   DevBuf off, list, woff, mem;
   DevArena work;
-  DevView cap, stamp, small, scan, cls, cnt;  // cnt: sizes, starts, fills
+  // cnt: list sizes, the first row with offsets, starts, fills.
+  DevView cap, stamp, small, scan, cls, cnt;
   work.add(cap, n1 * 8);
   work.add(stamp, size_t(c.groups) * below * 4);
   work.add(small, kSmallBytes);
@@ -436,7 +438,6 @@ int pairs_layout(mgpm_dgraph *dg, hipStream_t s) {
   work.add(cls, n0);
   work.add(cnt, kCls);
   MGPM_HIP(off.alloc(n1 * 8));
-  MGPM_HIP(woff.alloc(n0 * (c.nf + 1) * sizeof(uint16_t)));
   MGPM_HIP(work.alloc(mem));
   c.stamp = stamp.as<uint32_t>();
   c.tab_cap = cap.as<unsigned long long>();
@@ -448,10 +449,9 @@ int pairs_layout(mgpm_dgraph *dg, hipStream_t s) {
     return rc;
   if ((rc = zero(cap.p, n1 * 8, s))) return rc;
   if ((rc = zero(cnt.p, kCls, s))) return rc;
-  if (census5_classes(c, cls.as<int8_t>(), sizes_d, s) ||
-      census5_window_offsets(c, woff.as<uint16_t>(), dg->cus, s))
+  if (census5_classes(c, cls.as<int8_t>(), sizes_d, s))
     return fail(MGPM_ERR_HIP, "census kernel launch failed");
-  unsigned sizes[kC5Lists], starts[kC5Lists];
+  unsigned sizes[kC5Lists + 1], starts[kC5Lists];
   MGPM_HIP(hipMemcpyAsync(sizes, sizes_d, sizeof(sizes),
                           hipMemcpyDeviceToHost, s));
   MGPM_HIP(hipStreamSynchronize(s));
@@ -462,10 +462,18 @@ int pairs_layout(mgpm_dgraph *dg, hipStream_t s) {
   }
   MGPM_HIP(list.alloc(std::max<size_t>(at, 1) * sizeof(int32_t)));
   c.anchors = list.as<int32_t>();
-  MGPM_HIP(hipMemcpyAsync(sizes_d + kC5Lists, starts, sizeof(starts),
+  c.first = static_cast<int32_t>(sizes[kC5Lists]);
+  // Only the anchors whose targets take LDS windows read the offsets.
+  if (starts[kC5Lists - 1] > starts[kC5Light + 1]) {
+    MGPM_HIP(woff.alloc((n1 - c.first) * (c.nf + 1) * sizeof(uint16_t)));
+    if (census5_window_offsets(c, woff.as<uint16_t>(), dg->cus, s))
+      return fail(MGPM_ERR_HIP, "census kernel launch failed");
+  }
+  unsigned *starts_d = sizes_d + kC5Lists + 1;
+  MGPM_HIP(hipMemcpyAsync(starts_d, starts, sizeof(starts),
                           hipMemcpyHostToDevice, s));
-  if (census5_lists(n, cls.as<int8_t>(), sizes_d + kC5Lists,
-                    sizes_d + 2 * kC5Lists, list.as<int32_t>(), s) ||
+  if (census5_lists(n, cls.as<int8_t>(), starts_d, starts_d + kC5Lists,
+                    list.as<int32_t>(), s) ||
       census5_table_count_launch(c, sizes, dg->cus, s))
     return fail(MGPM_ERR_HIP, "census kernel launch failed");
   if (census5_scan(cap.as<unsigned long long>(), off.as<unsigned long long>(),
@@ -476,6 +484,7 @@ int pairs_layout(mgpm_dgraph *dg, hipStream_t s) {
                           hipMemcpyDeviceToHost, s));
   MGPM_HIP(hipStreamSynchronize(s));  // the work arrays die here
   for (int k = 0; k < kC5Lists; ++k) cg.c5_count[k] = sizes[k];
+  cg.c5_first = c.first;
   cg.tab_off.swap(off);
   cg.c5_list.swap(list);
   cg.c5_woff.swap(woff);

@@ -162,10 +162,13 @@ struct Census5Args {
   const unsigned long long *tv = nullptr;  // twice the triangles per vertex
   const uint32_t *arc = nullptr;     // DAG arc of every CSR entry
   const int32_t *anchors = nullptr;  // the lists of anchors, in order
-  // The window: its lowest id, the first entry of every row in it, and per
-  // row the entries before each of nf fine windows (nf + 1 per row).
+  // The window: its lowest id, the first entry of every row in it, and the
+  // entries of a row before each of nf fine windows (nf + 1 per row): zeros
+  // for the rows below `first`, the first vertex of two neighbours (one of a
+  // single neighbour leads only back to the anchor), then a row each.
   int32_t winlo = 0;
   int nf = 0;
+  int32_t first = 0;
   const uint32_t *win = nullptr;
   const uint16_t *woff = nullptr;
   // Per workgroup, for the targets below the window (or, last list, all):
@@ -197,13 +200,13 @@ int census5_flat_launch(const Census5Args &c, int cus, hipStream_t s);
 int census5_table_count_launch(const Census5Args &c, const uint32_t *count,
                                int cus, hipStream_t s);
 // The anchors' lists: classes of all vertices (n; list sizes into fill,
-// kC5Lists entries, zeroed), then, with fill zeroed again and the starts of
+// kC5Lists entries, zeroed, and Census5Args::first after them), then, with fill zeroed again and the starts of
 // the lists, the lists.
 int census5_classes(const Census5Args &c, int8_t *cls, unsigned *fill,
                     hipStream_t s);
 int census5_lists(int32_t n, const int8_t *cls, const unsigned *start,
                   unsigned *fill, int32_t *list, hipStream_t s);
-// Fine windows of a graph, and the offsets of every row (n x (nf + 1)).
+// Fine windows of a graph, and their offsets (n - first + 1 rows of nf + 1).
 int census5_fine_windows(int32_t n, int32_t winlo);
 int census5_window_offsets(const Census5Args &c, uint16_t *woff, int cus,
                            hipStream_t s);

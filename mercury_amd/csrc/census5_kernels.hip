@@ -196,6 +196,22 @@ __global__ __launch_bounds__(kClassT) void c5_scatter(
   }
 }
 
+// The first vertex of at least two neighbours (ids are ranks by degree).
+__global__ void c5_first(Census5Args c, unsigned *__restrict__ first) {
+  int32_t lo = 0, hi = c.n;
+  while (lo < hi) {
+    const int32_t mid = lo + (hi - lo) / 2;
+    if (c.deg[mid] < 2) lo = mid + 1;
+    else hi = mid;
+  }
+  *first = static_cast<unsigned>(lo);
+}
+
+// The row of vertex v in the fine windows' offsets.
+__device__ __forceinline__ int64_t woff_row(const Census5Args &c, int32_t v) {
+  return max(v - c.first, -1) + 1;
+}
+
 // First entry of every row in each of the nf fine windows (kFine ids each
 // from winlo), relative to the row's first entry in the window; entry nf:
 // the row's entries in the window.  One thread per entry fills the windows
@@ -208,18 +224,21 @@ __global__ void c5_window_offsets(Census5Args c, uint16_t *__restrict__ woff) {
     const int32_t u = c.col[j];
     if (u < c.winlo) continue;
     const int32_t v = c.src[j];
+    if (v < c.first) continue;
     const int64_t w = c.win[v];
     const int f = (u - c.winlo) / kFine;
     const int from = j == w ? 0 : (c.col[j - 1] - c.winlo) / kFine + 1;
     for (int g = from; g <= f; ++g)
-      woff[int64_t(v) * stride + g] = static_cast<uint16_t>(j - w);
+      woff[woff_row(c, v) * stride + g] = static_cast<uint16_t>(j - w);
   }
-  for (int64_t v = i0; v < c.n; v += step) {
+  for (int64_t v = c.first + i0; v < c.n; v += step) {
     const int64_t w = c.win[v], e = c.rowptr[v + 1];
     const int from = e > w ? (c.col[e - 1] - c.winlo) / kFine + 1 : 0;
     for (int g = from; g <= c.nf; ++g)
-      woff[v * stride + g] = static_cast<uint16_t>(e - w);
+      woff[woff_row(c, static_cast<int32_t>(v)) * stride + g] =
+          static_cast<uint16_t>(e - w);
   }
+  if (i0 <= c.nf) woff[i0] = 0;
 }
 
 // Adjacency bit rows of G[N+(a)]: bit j of row i iff nb[j] ~ nb[i].
@@ -512,7 +531,7 @@ __device__ __forceinline__ bool add_window(const Census5Args &c, int32_t a,
     uint32_t b = 0, len = 0;
     if (k < d) {
       const int32_t y = c.col[rb + k];
-      const uint16_t *wo = c.woff + y * stride;
+      const uint16_t *wo = c.woff + woff_row(c, y) * stride;
       b = c.win[y] + wo[f0];
       len = uint32_t(wo[f1]) - wo[f0];
     }
@@ -1074,6 +1093,7 @@ int census5_classes(const Census5Args &c, int8_t *cls, unsigned *fill,
   hipLaunchKernelGGL(c5_classes, dim3(g), dim3(256), 0, s, c, cls);
   hipLaunchKernelGGL(c5_scatter, dim3(c.n / kClassT + 1), dim3(kClassT), 0, s,
                      cls, c.n, nullptr, fill, nullptr);
+  hipLaunchKernelGGL(c5_first, dim3(1), dim3(1), 0, s, c, fill + kC5Lists);
   return hipGetLastError() == hipSuccess ? 0 : -1;
 }
 

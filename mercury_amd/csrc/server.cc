@@ -298,6 +298,10 @@ int mgpm_server_add_graph(mgpm_server *s, const mgpm_graph *g,
     if ((rc = mgpm_dgraph_upload(g, s->cfg.device, nullptr, &dg))) return rc;
     if (s->cfg.pattern_census >= 0) {
       rc = census_graph_prepare(dg, nullptr);
+      if (!rc) {  // every count reads the relabelled copy from here on
+        dg->csr.rowptr.reset();
+        dg->csr.colidx.reset();
+      }
     } else {
       for (int p = MGPM_P1; p <= MGPM_P8 && !rc; ++p)
         rc = pattern_make_resident(dg, nullptr, p);

@@ -1,6 +1,7 @@
 """The server's budget and the hub plans of triangle counts: a plan is kept
 where there is room for it and gives its memory back to a graph or a request
 that needs it, so that what fits without the plans is served."""
+import numpy as np
 import pytest
 
 import mercury_amd as ma
@@ -91,3 +92,43 @@ def test_request_takes_the_room_of_a_hub_plan(gpu_available, sizes):
     assert srv.stats().resident_bytes == sizes["base"]
     assert _count(srv, gid, 0) == sizes["tc"]
     srv.close()
+
+
+def test_graph_keeps_no_more_than_its_plans(gpu_available):
+    """Beside the uploaded graph and its triangle plan, 12 bytes per CSR entry
+    and 28 per vertex: the windows' offsets leave out vertices of one
+    neighbour, and the uploaded CSR goes when its relabelled copy is there."""
+    g = ma.Graph.rmat(17, 16, seed=4)
+    dg = ma.DeviceGraph(g, 0)
+    plans = dg.footprint()
+    dg.pattern_count(2)
+    before = dg.footprint()
+    dg.tc_count()
+    hub = dg.footprint() - before
+    dg.close()
+    srv = ma.Server(0)
+    gid = srv.add_graph(g)
+    kept = srv.stats().resident_bytes - hub
+    assert kept <= plans + 12 * g.nnz + 28 * (g.n + 1)
+    assert _count(srv, gid, 0) > 0
+    srv.close()
+
+
+def test_window_offsets_of_few_neighbours(gpu_available):
+    """Heavy anchors whose neighbours have one neighbour, two or many."""
+    rows, hubs, n = [], 6, 6 + 3000
+    for h in range(hubs):  # a clique; leaf v hangs on hubs v % 6 (and v + 1)
+        rows.append([x for x in range(hubs) if x != h])
+    for v in range(hubs, n):
+        mine = sorted({v % hubs, (v + 1) % hubs} if v % 3 == 0 else {v % hubs})
+        rows.append(mine)
+        for h in mine:
+            rows[h].append(v)
+    rp = np.zeros(n + 1, dtype=np.int64)
+    rp[1:] = np.cumsum([len(r) for r in rows])
+    g = ma.Graph.from_csr(rp, np.concatenate(rows).astype(np.int32))
+    dg = ma.DeviceGraph(g, 0)
+    for p in (2, 3, 5, 6):
+        assert dg.pattern_count(p)[0] == dg.pattern_count(
+            p, ma.make_tune(pattern_census=-1))[0], p
+    dg.close()
