@@ -104,7 +104,7 @@ size_t row_slab(const mgpm_dgraph *dg, int passes, int64_t max_out,
   for (int cls = 0; cls < kRowClassCount; ++cls)
     for (const bool cliques : {false, true})
       if (cliques ? is_k5(passes) : cls == kRowClassCount - 1)
-        b = std::max(b, rows_slab_bytes(cls, max_out) *
+        b = std::max(b, rows_slab_bytes(cls, max_out, cliques) *
                             rows_grid(cls, max_out,
                                       count ? rows_members(cls, count, cliques)
                                             : dg->host->n,

@@ -231,7 +231,7 @@ int census_rows_init();
 // Slab bytes per workgroup of class `cls`, and its workgroups (0 for an
 // empty class) within `budget` bytes of slab, for graphs whose largest DAG
 // out-degree is max_out.  cliques: the pass of that setting.
-size_t rows_slab_bytes(int cls, int64_t max_out);
+size_t rows_slab_bytes(int cls, int64_t max_out, bool cliques);
 // Vertices of class `cls` in a pass, of the class sizes count.
 int64_t rows_members(int cls, const int64_t *count, bool cliques);
 int rows_grid(int cls, int64_t max_out, int64_t count, bool cliques,
