@@ -40,7 +40,9 @@ class BatchExec {
   // Device bytes plan() may add to the workspaces for these queries (a
   // bound: every lane grown to the largest query's needs; 0 if they fit
   // what is there).  query_need folds one query into the running maxima
-  // that growth_for turns into that bound, for callers growing a set.
+  // that growth_for turns into that bound, for callers growing a set.  Hub
+  // plans are not in it: a caller with a bound builds them with its graphs,
+  // or refuses them (server.cc), and plan() adds none.
   uint64_t growth(const mgpm_query *q, int nq) const;
   void query_need(const mgpm_query &q, uint64_t *want_census,
                   uint64_t *want_slab) const;

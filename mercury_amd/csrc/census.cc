@@ -323,10 +323,15 @@ unsigned long long *census_acc(const CensusWork &w) {
 uint64_t census_work_bytes(const mgpm_dgraph *dg, int passes,
                            size_t budget) {
   if (!dg->census.ready) {
-    // The DAG the graph will keep, plus a bound on the workspace.
+    // What the graph will keep (a bound), plus a bound on the workspace.
     const CsrGraph &G = *dg->host;
-    const uint64_t dag = 8ull * G.n + 8ull * G.nnz + 8ull * (G.n + 1) +
-                         8ull * (G.nnz / 2);
+    const uint64_t n1 = static_cast<uint64_t>(G.n) + 1;
+    uint64_t dag = 24ull * n1 + 14ull * G.nnz;  // the census graph
+    if (needs_c4(passes)) dag += 16ull * n1;    // windows, three lists
+    if (is_full5(passes)) {                     // table, list, offsets
+      const int32_t winlo = std::max<int32_t>(0, G.n - kRowWindow);
+      dag += (12ull + 2ull * (census5_fine_windows(G.n, winlo) + 1)) * n1;
+    }
     const uint64_t work = is_full5(passes) ? budget + 16ull * G.nnz
                                            : 32ull * G.nnz;
     return dag + work +
