@@ -318,9 +318,11 @@ int mgpm_pattern_count_noalloc(mgpm_dgraph *dg, int pattern, void *stream,
  * the device (median kernel time of `reps` runs, 0 = 3) and must return the
  * same count as the starting point (MGPM_ERR_INTERNAL otherwise).  The
  * winner stays resident on the graph -- later calls with a NULL tune,
- * batches and servers use it, or the hub bitmaps of mgpm_tc_count where
- * those measure faster -- and is returned in *best (may be NULL)
- * with its time in *best_ms (may be NULL). */
+ * batches and servers use it -- and is returned in *best (may be NULL)
+ * with its time in *best_ms (may be NULL).  MGPM_TC: where the hub bitmaps
+ * of mgpm_tc_count measure faster than every table plan, they are the
+ * winner: NULL and *best count against them on this handle, *best_ms is
+ * their time, and the knobs in *best are the best table plan's. */
 int mgpm_autotune(mgpm_dgraph *dg, int pattern, int32_t reps, mgpm_tune *best,
                   double *best_ms);
 

@@ -81,6 +81,7 @@ int tune_tc(mgpm_dgraph *dg, int reps, mgpm_tune *best, double *best_ms) {
   mgpm_tune cur = tune_of(dg->tc);
   uint64_t want = 0;
   double cur_ms = 0;
+  dg->hub.has_best = false;  // every tune below is timed on the tables
   int rc = time_tc(dg, cur, reps, &want, &cur_ms);
   if (rc) return rc;
   const std::vector<Knob> knobs = {
@@ -124,8 +125,8 @@ int tune_tc(mgpm_dgraph *dg, int reps, mgpm_tune *best, double *best_ms) {
   dg->tc.tuned = true;
   *best = cur;
   *best_ms = cur_ms;
-  // Counts with a NULL tune stay on the hub bitmaps unless the tuned table
-  // plan beats them.
+  // Counts with a NULL tune, or the one returned, stay on the hub bitmaps
+  // unless the tuned table plan beats them.
   dg->hub.off = false;
   if (tc_hub_wanted(dg)) {
     std::vector<double> k;
@@ -135,9 +136,16 @@ int tune_tc(mgpm_dgraph *dg, int reps, mgpm_tune *best, double *best_ms) {
       if ((rc = mgpm_tc_count(dg, nullptr, nullptr, &c, &st))) return rc;
       if (c != want)
         return fail(MGPM_ERR_INTERNAL, "autotune: candidate count differs");
+      if (st.path != 3) return MGPM_OK;  // no memory for the hub plan
       if (i > 0) k.push_back(st.kernel_ms);
     }
-    dg->hub.off = cur_ms < 0.98 * median(k);
+    const double hub_ms = median(k);
+    dg->hub.off = cur_ms < 0.98 * hub_ms;
+    if (!dg->hub.off) {
+      dg->hub.best = cur;
+      dg->hub.has_best = true;
+      *best_ms = hub_ms;
+    }
   }
   return MGPM_OK;
 }

@@ -5,6 +5,7 @@
 #include <atomic>
 #include <cstring>
 #include <new>
+#include <tuple>
 
 #include "capi_common.hpp"
 #include "census.hpp"
@@ -195,12 +196,19 @@ int set_device(int device) {
 
 const char *last_error_cstr() { return g_last_error.c_str(); }
 
-// Whether a tune sets a field that the table plan or its launch reads.
-bool tc_knob_set(const mgpm_tune *t) {
-  return t && (t->small_max_deg || t->wave_max_deg || t->block_max_deg ||
-               t->chunk_work || t->grid_blocks || t->group_work ||
-               t->tc_items || t->tc_cursor_min || t->tc_layout ||
-               t->tc_merge_max || t->tc_half_waves);
+// The fields of a tune that the table plan or its launch reads.
+auto tc_knobs(const mgpm_tune &t) {
+  return std::make_tuple(t.small_max_deg, t.wave_max_deg, t.block_max_deg,
+                         t.chunk_work, t.grid_blocks, t.group_work, t.tc_items,
+                         t.tc_cursor_min, t.tc_layout, t.tc_merge_max,
+                         t.tc_half_waves);
+}
+
+// Whether a tune asks for the table plan: one that sets any of them, but for
+// the autotuner's own answer where the hub bitmaps beat it.
+bool tc_tables_asked(const TcHub &h, const mgpm_tune *t) {
+  return t && tc_knobs(*t) != tc_knobs(mgpm_tune{}) &&
+         !(h.has_best && tc_knobs(*t) == tc_knobs(h.best));
 }
 
 // What follows a triangle count's launches (enqueued after dg->ev0): the
@@ -600,7 +608,7 @@ int mgpm_tc_count(mgpm_dgraph *dg, const mgpm_tune *tune, void *stream,
   // Hub bitmaps where hubs dominate, unless a triangle knob asks for the
   // table plan; the plan is built on the first such count.
   bool hub = false;
-  if (!tc_knob_set(tune)) {
+  if (!tc_tables_asked(dg->hub, tune)) {
     const bool had = dg->hub.ready;
     if ((rc = tc_hub_use(dg, s, &hub))) return rc;
     if (hub && !had) prep = ms_since(t0);

@@ -220,6 +220,10 @@ struct CensusGraph {
 struct TcHub {
   std::atomic<int> wanted{-1};  // the rule's answer (-1: not asked yet)
   bool off = false;  // the autotuner measured a table plan as faster
+  // What the autotuner returned where the hub bitmaps are faster: passed back
+  // it takes them, as a null tune does.
+  bool has_best = false;
+  mgpm_tune best{};
   bool refused = false;  // its server has no memory for it
   size_t short_of = 0;  // free device bytes when it could not be allocated
   std::atomic<bool> ready{false};
