@@ -131,9 +131,15 @@ typedef struct mgpm_stats {
   uint64_t m;         /* undirected edges */
   uint64_t m_plus;    /* DAG arcs (TC) */
   uint64_t s_plus;    /* sum over DAG arcs u->v of d+(v) (TC wedge checks) */
-  uint64_t probes;    /* TC: hash probes issued by the chosen schedule */
-  uint64_t bytes_alg; /* TC: 8(n+1) + 20 m+ + 4 S+ */
-  int32_t path;       /* implementation path id (diagnostic) */
+  uint64_t probes;    /* TC: hash probes issued by the chosen schedule (path
+                         3: ids tested against the bitmaps, with the padding
+                         of the rows' chunks) */
+  uint64_t bytes_alg; /* TC: 8(n+1) + 20 m+ + 4 S+ (path 3: the owners'
+                         records and rows once, every partner's record and
+                         the chunks of its row past the owner) */
+  int32_t path;       /* implementation path id (diagnostic): TC 1 = hash
+                         tables, lists gathered; 2 = laid-out lists; 3 = hub
+                         bitmaps */
   int32_t reserved[3];
 } mgpm_stats;
 

@@ -232,9 +232,17 @@ int tc_finish(mgpm_dgraph *dg, hipStream_t s,
     stats->m = static_cast<uint64_t>(dg->host->nnz / 2);
     stats->m_plus = dg->tc.m_plus;
     stats->s_plus = dg->tc.s_plus;
-    stats->probes = dg->tc.probes;
-    stats->bytes_alg =
-        8ull * (stats->n + 1) + 20ull * stats->m_plus + 4ull * stats->s_plus;
+    if (path == 3) {
+      const TcHub &h = dg->hub;
+      stats->probes = kHubChunk * h.part_chunks;
+      stats->bytes_alg = sizeof(HubOwner) * uint64_t(h.plan.owners) +
+                         sizeof(HubPartner) * uint64_t(h.plan.nparts) +
+                         2ull * kHubChunk * (h.part_chunks + h.row_chunks);
+    } else {
+      stats->probes = dg->tc.probes;
+      stats->bytes_alg =
+          8ull * (stats->n + 1) + 20ull * stats->m_plus + 4ull * stats->s_plus;
+    }
     stats->path = path;
     stats->e2e_ms = ms_since(t0);
   }

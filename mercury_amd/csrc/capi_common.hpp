@@ -230,6 +230,8 @@ struct TcHub {
   TcHubPlan plan;
   DevBuf mem;   // everything plan points at, and own
   DevView own;  // result and queue of single counts (zero between them)
+  // Chunks a count reads: of the partners' rows, and the owners' rows.
+  uint64_t part_chunks = 0, row_chunks = 0;
   size_t bytes() const { return mem.bytes; }
 };
 

@@ -506,31 +506,55 @@ __global__ void hub_partners(const int32_t *__restrict__ col,
   }
 }
 
+// Adds a workgroup's sum to one of the kHubSums places.
+__device__ __forceinline__ void add_sum(u64 x, u64 *__restrict__ sums) {
+  __shared__ u64 s_sum;
+  if (threadIdx.x == 0) s_sum = 0;
+  __syncthreads();
+  x = wave_sum_u64(x);
+  if (lane64() == 0) atomicAdd(&s_sum, x);
+  __syncthreads();
+  if (threadIdx.x == 0 && s_sum)
+    atomicAdd(&sums[blockIdx.x % kHubSums * kHubSumStride], s_sum);
+}
+
 // Cost of every run of kHubRun partners, in steps of one group of lanes,
 // with kOwnerCost more where an owner with a row begins (hub_owner_costs).
+// Both also add up the chunks that a count reads.
 __global__ void hub_costs(const HubPartner *__restrict__ part,
                           uint32_t nparts, uint32_t runs,
-                          u64 *__restrict__ cost) {
+                          u64 *__restrict__ cost, u64 *__restrict__ sums) {
   static_assert(kHubRun == 16, "a run per 16 lanes");
+  u64 chunks = 0;
   const uint32_t gl = threadIdx.x % kHubRun;
   for (uint32_t r = (blockIdx.x * blockDim.x + threadIdx.x) / kHubRun;
        r <= runs; r += gridDim.x * blockDim.x / kHubRun) {
     const uint32_t i = r * kHubRun + gl;
     int c = 0;
-    if (r < runs && i < nparts)
-      c = static_cast<int>(max(1u, (part[i].chunks + kLanes - 1u) / kLanes));
+    if (r < runs && i < nparts) {
+      const uint32_t k = part[i].chunks;
+      chunks += k;
+      c = static_cast<int>(max(1u, (k + kLanes - 1u) / kLanes));
+    }
 #pragma unroll
     for (int d = 8; d >= 1; d >>= 1) c += __shfl_xor(c, d, 16);
     if (gl == 0) cost[r] = static_cast<u64>(c);
   }
+  add_sum(chunks, sums);
 }
 
 __global__ void hub_owner_costs(const HubOwner *__restrict__ owner,
                                 const uint32_t *__restrict__ owners,
-                                u64 *__restrict__ cost) {
+                                u64 *__restrict__ cost,
+                                u64 *__restrict__ sums) {
+  u64 chunks = 0;
   for (uint32_t k = blockIdx.x * blockDim.x + threadIdx.x; k < *owners;
-       k += gridDim.x * blockDim.x)
-    atomicAdd(&cost[owner[k].beg / kHubRun], kOwnerCost);
+       k += gridDim.x * blockDim.x) {
+    const HubOwner o = owner[k];
+    chunks += o.chunks;
+    atomicAdd(&cost[o.beg / kHubRun], kOwnerCost);
+  }
+  add_sum(chunks, sums + 1);
 }
 
 // Block g holds the runs whose cost prefix starts in [g, g + 1) / blocks of
@@ -642,12 +666,12 @@ int tc_hub_scan(const uint32_t *chunks, uint32_t *rowbase, int32_t n,
 int tc_hub_blocks(const TcHubPlan &p, const uint32_t *owners, uint32_t runs,
                   unsigned long long *cost, unsigned long long *prefix,
                   void *tmp, size_t bytes, uint32_t *bound, uint32_t *start,
-                  hipStream_t s) {
+                  unsigned long long *sums, hipStream_t s) {
   hipLaunchKernelGGL(hub_costs, dim3(flat((int64_t(runs) + 1) * kHubRun,
                                           8192)),
-                     dim3(256), 0, s, p.part, p.nparts, runs, cost);
+                     dim3(256), 0, s, p.part, p.nparts, runs, cost, sums);
   hipLaunchKernelGGL(hub_owner_costs, dim3(flat(p.n, 4096)), dim3(256), 0, s,
-                     p.owner, owners, cost);
+                     p.owner, owners, cost, sums);
   if (hipcub::DeviceScan::ExclusiveSum(tmp, bytes, cost, prefix,
                                        int64_t(runs) + 1, s) != hipSuccess)
     return -1;

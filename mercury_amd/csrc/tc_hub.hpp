@@ -65,12 +65,17 @@ struct HubOut {
 int tc_hub_launch(const TcHubPlan &p, const HubOut &out, int cus,
                   hipStream_t s);
 
+// The chunks that a plan names, added up in kHubSums places, kHubSumStride
+// 64-bit words apart: of the partners, then of the owners' rows.
+constexpr int kHubSums = 16;
+constexpr int kHubSumStride = 16;
+
 // Preparation: split (n) and the chunks of every row (n + 1, the last 0);
 // the caller scans them into rowbase, then the rows, owners (flag and pos
 // hold n + 1 entries, pos[n] their number; meta 16 bytes per vertex),
 // partners and the rest list
 // (its size into *nrest, zeroed), then the blocks (runs = ceil(nparts /
-// kHubRun); cost and prefix hold runs + 1 entries).
+// kHubRun); cost and prefix hold runs + 1 entries; sums zeroed).
 int tc_hub_counts(const int64_t *drp, const int32_t *dcol, int32_t n,
                   int32_t hublo, uint32_t *split, uint32_t *chunks,
                   hipStream_t s);
@@ -87,6 +92,6 @@ int tc_hub_fill(const int64_t *rowptr, const int32_t *col,
 int tc_hub_blocks(const TcHubPlan &p, const uint32_t *owners, uint32_t runs,
                   unsigned long long *cost, unsigned long long *prefix,
                   void *tmp, size_t bytes, uint32_t *bound, uint32_t *start,
-                  hipStream_t s);
+                  unsigned long long *sums, hipStream_t s);
 
 }  // namespace mgpm
