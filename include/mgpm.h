@@ -109,7 +109,11 @@ typedef struct mgpm_tune {
                              the plan: 4 bytes per probe + 8 per partner),
                              -1 = gather them from the DAG; 0 (default) =
                              lay out when the copy fits a quarter of the
-                             free device memory.  Same count either way. */
+                             free device memory.  Same count either way.
+                             Lists are only laid out for counts on the hash
+                             tables: where hubs dominate, a count without
+                             triangle knobs goes against hub bitmaps and
+                             builds their plan instead. */
   int32_t tc_merge_max;   /* TC: owners with d+ up to this (at most 64)
                              skip the hash table: each lane merges one
                              partner list with the owner's sorted list (two

@@ -30,8 +30,8 @@
 // 4.4e9 + 1.2e9 items and intersects 9.6e9 word pairs.  Measured on one
 // MI355X against one wave per DAG arc with binary searches (arcs from one
 // atomic cursor, 11 ns each): t and 4-cliques at RMAT-20 329 -> 7.3 ms;
-// P7 at RMAT-18 280 -> 8.3 ms; P1 on 300007 vertices of degree 16
-// (2.4 million arcs) 27.4 -> 0.79 ms.  Before the vertices with many lower
+// P7 at RMAT-18 280 -> 8.0 ms; P1 on 300007 vertices of degree 16
+// (2.4 million arcs) 27.4 -> 0.26 ms (census_tiny).  Before the vertices with many lower
 // neighbours went to the large workgroups and the ranges were loaded 16 at a
 // time, 20.3 and 17.9 ms.
 #include <hip/hip_runtime.h>

@@ -64,7 +64,12 @@ bool hubs_hold(const CsrGraph &g, int64_t num, int64_t den) {
 //   beyond, where the hubs hold half of all degrees (uniform graphs: 150001
 //   vertices 142 / 146, 200003 vertices 262 / 181), or a quarter and the
 //   lists that the tables would stream average 32 items or more, which a
-//   hash probe each makes dear (RMAT-22: 3650 / 15700).
+//   hash probe each makes dear (RMAT-22: 3600 / 15800).
+// These are the counts of a resident plan.  A handle's first count also builds
+// it, from the census graph (ms, bitmaps / laid-out tables): RMAT-11 0.38 /
+// 0.16, RMAT-12 0.43 / 0.21, RMAT-14 0.62 / 0.44, RMAT-15 0.72 / 0.76, RMAT-16
+// 0.85 / 1.05, RMAT-18 1.74 / 2.35: below about 300000 arcs 0.2 ms more, which
+// one to ten further counts give back.
 bool hubs_pay(const mgpm_dgraph *dg) {
   const CsrGraph &g = *dg->host;
   if (g.nnz / 2 < 16384 || g.nnz >= (int64_t(1) << 32)) return false;

@@ -25,12 +25,13 @@
 // Triangles without a hub (both lists short) are found by binary search
 // (hub_rest).
 //
-// Measured on one MI355X, per count: RMAT-22 (16 draws per vertex) 15.7 ms
-// with hash tables on laid-out lists -> 3.65 ms (hub_count 3.0, hub_rest
-// 0.6), with 1.9 GB of plan instead of 48 GB; RMAT-16 705 -> 67 us.  What
-// bounds it: the rows come from the last-level cache (20 GB per count on
-// RMAT-22 at 6.5 TB/s: the L2 catches a sixth), 73 vector instructions and
-// eight LDS reads per step of 512 items behind that.
+// Measured on one MI355X, per count: RMAT-22 (16 draws per vertex) 15.8 ms
+// with hash tables on laid-out lists -> 3.6 ms (hub_count 3.0, hub_rest
+// 0.69), with 0.8 GB of plan beside the census graph's 1.9 GB instead of 48
+// GB of lists; RMAT-16 708 -> 67 us.  What bounds it: the rows come from the
+// last-level cache (20 GB per count on RMAT-22 at 6.5 TB/s: the L2 catches a
+// sixth; the plan names 15.4 GB of records and chunks), 73 vector instructions
+// and eight LDS reads per step of 512 items behind that.
 #include <hip/hip_runtime.h>
 
 #include <hipcub/device/device_scan.hpp>
