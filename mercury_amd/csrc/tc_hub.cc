@@ -125,7 +125,7 @@ int prepare(mgpm_dgraph *dg, hipStream_t s) {
   DevArena keep;
   keep_layout(dg, p, k, keep);
   DevBuf mem, tmp_mem;  // mem becomes h.mem when it is complete
-  DevView rowbase, chunks, flag, pos, meta, cost, prefix, total, sums, scan;
+  DevView rowbase, chunks, flag, pos, meta, cost, prefix, sums, scan;
   const size_t sb = tc_hub_scan_bytes(n, runs);
   if (sb == 0) return fail(MGPM_ERR_HIP, "scan size query");
   DevArena work;
@@ -133,8 +133,9 @@ int prepare(mgpm_dgraph *dg, hipStream_t s) {
   work.add(meta, n1 * 16);
   work.add(cost, (size_t(runs) + 1) * 8);
   work.add(prefix, (size_t(runs) + 1) * 8);
+  // The sums of chunks, and in the first place's third word the rest's size:
+  // one fill, one copy back.
   constexpr size_t kSums = size_t(kHubSums) * kHubSumStride;
-  work.add(total, 4);
   work.add(sums, kSums * 8);
   work.add(scan, sb);
   MGPM_HIP(keep.alloc(mem));
@@ -149,38 +150,38 @@ int prepare(mgpm_dgraph *dg, hipStream_t s) {
   p.dcol = dcol;
   p.split = k.split.as<uint32_t>();
   const uint32_t *owners = pos.as<uint32_t>() + n;
+  uint32_t *nrest =
+      reinterpret_cast<uint32_t *>(sums.as<unsigned long long>() + 2);
   if (tc_hub_counts(drp, dcol, n, hublo, k.split.as<uint32_t>(),
                     chunks.as<uint32_t>(), s) ||
       tc_hub_scan(chunks.as<uint32_t>(), rowbase.as<uint32_t>(), n, scan.p,
                   sb, s) ||
-      device_zero(total.p, 1, s) || device_zero(sums.p, 2 * kSums, s) ||
-      device_zero(k.own.p, kOwnWords, s) ||
+      device_zero(sums.p, 2 * kSums, s) || device_zero(k.own.p, kOwnWords, s) ||
       tc_hub_fill(cg.rowptr.as<int64_t>(), cg.col.as<int32_t>(),
                   cg.src.as<int32_t>(), nnz, drp, dcol, cg.arc.as<uint32_t>(),
                   n, k.split.as<uint32_t>(), rowbase.as<uint32_t>(), k.rows.p,
                   flag.as<uint32_t>(), pos.as<uint32_t>(), meta.p,
                   k.owner.as<HubOwner>(), k.part.as<HubPartner>(),
-                  k.rest.as<int32_t>(), total.as<uint32_t>(), scan.p, sb,
+                  k.rest.as<int32_t>(), nrest, scan.p, sb,
                   dg->cus, s) ||
       tc_hub_blocks(p, owners, runs, cost.as<unsigned long long>(),
                     prefix.as<unsigned long long>(), scan.p, sb,
                     k.bound.as<uint32_t>(), k.start.as<uint32_t>(),
                     sums.as<unsigned long long>(), s))
     return fail(MGPM_ERR_HIP, "hub plan kernel launch failed");
-  MGPM_HIP(hipMemcpyAsync(&p.nrest, total.p, 4, hipMemcpyDeviceToHost, s));
   MGPM_HIP(hipMemcpyAsync(&p.owners, owners, 4, hipMemcpyDeviceToHost, s));
-  unsigned long long chunks_read[kSums];
-  MGPM_HIP(hipMemcpyAsync(chunks_read, sums.p, sizeof(chunks_read),
-                          hipMemcpyDeviceToHost, s));
+  unsigned long long got[kSums];
+  MGPM_HIP(hipMemcpyAsync(got, sums.p, sizeof(got), hipMemcpyDeviceToHost, s));
   MGPM_HIP(hipStreamSynchronize(s));  // the work arrays die here
+  p.nrest = static_cast<uint32_t>(got[2]);
   if (p.owners == 0) p.blocks = 0;  // no arc follows another: no triangle
   h.mem.swap(mem);
   h.plan = p;
   h.own = k.own;
   h.part_chunks = h.row_chunks = 0;
   for (int i = 0; i < kHubSums; ++i) {
-    h.part_chunks += chunks_read[i * kHubSumStride];
-    h.row_chunks += chunks_read[i * kHubSumStride + 1];
+    h.part_chunks += got[i * kHubSumStride];
+    h.row_chunks += got[i * kHubSumStride + 1];
   }
   h.ready = true;
   return MGPM_OK;
