@@ -114,8 +114,8 @@ bool hub_in_flight(const mgpm_server *s, int32_t gid) {
 }
 
 // Hub plans take memory that nothing else needs: frees those that no batch
-// in flight uses until `bytes` fit the budget, and keeps new batches off the
-// others (lock held).  Returns whether the bytes fit.
+// in flight uses until `bytes` fit the budget, and if they do not, keeps new
+// batches off the others (lock held).  Returns whether the bytes fit.
 bool make_room(mgpm_server *s, uint64_t bytes) {
   uint64_t hubs = 0;
   for (const mgpm_dgraph *g : s->graphs) hubs += g->hub.bytes();
@@ -123,13 +123,13 @@ bool make_room(mgpm_server *s, uint64_t bytes) {
   for (size_t i = 0; i < s->graphs.size() && bytes > room_for(s); ++i) {
     mgpm_dgraph *g = s->graphs[i];
     const uint64_t b = g->hub.bytes();
-    if (!b) continue;
-    g->hub.refused = true;
-    if (hub_in_flight(s, static_cast<int32_t>(i))) continue;
+    if (!b || hub_in_flight(s, static_cast<int32_t>(i))) continue;
     tc_hub_release(g);
     s->resident -= b;
   }
-  return bytes <= room_for(s);
+  if (bytes <= room_for(s)) return true;
+  for (mgpm_dgraph *g : s->graphs) g->hub.refused = true;
+  return false;
 }
 
 // Takes pending requests in arrival order for free slot `sl` while their
@@ -313,15 +313,19 @@ int mgpm_server_add_graph(mgpm_server *s, const mgpm_graph *g,
     uint64_t bytes = 0;
     mgpm_dgraph_footprint(dg, &bytes);
     std::unique_lock<std::mutex> lk(s->mu);
-    while (bytes > room_for(s) && !make_room(s, bytes)) {
+    bool fits;
+    while (!(fits = bytes <= room_for(s) || make_room(s, bytes))) {
       // Hub plans in use go when their batches are done.
       uint64_t hubs = 0;
       for (const mgpm_dgraph *o : s->graphs) hubs += o->hub.bytes();
-      if (bytes > room_for(s) + hubs) {
-        mgpm_dgraph_free(dg);
-        return fail(MGPM_ERR_CAPACITY, "graph does not fit the HBM budget");
-      }
+      if (bytes > room_for(s) + hubs) break;
       s->cv_done.wait(lk);
+    }
+    for (mgpm_dgraph *o : s->graphs)  // plans that stay are used again
+      if (o->hub.ready) o->hub.refused = false;
+    if (!fits) {
+      mgpm_dgraph_free(dg);
+      return fail(MGPM_ERR_CAPACITY, "graph does not fit the HBM budget");
     }
     s->resident += bytes;
     uint64_t hub = 0;  // reserved while it is built
